@@ -198,8 +198,8 @@ def run(s):
 
 
 def work(case):
-    """Bytes: each point's position, strength and mode once. Operations: the kernel's taps and the pruned transform's
-    share of 5 n log2 n."""
+    """Bytes: each point's position, strength and mode once. Operations: the
+    kernel's taps and the pruned transform's share of 5 n log2 n."""
     eps, dim = case["eps"], case["dim"]
     if case["call"] == "t3":
         w = mn.kernel_params(eps, 1.25)[0]
@@ -223,10 +223,10 @@ def tolerance(case):
     """Four times what the same path was seen to differ by with its sums in
     another order (tiles instead of sweeps, full instead of pruned transform;
     in type 3 the gather along another axis): 32-bit weights, sums and
-    transforms give up to 7e-7. The modes
-    at the edge of the box are divided by the kernel's small transform there,
-    which at upsampling 1.25 raises that rounding to 3.2e-5 (3.1e-3 of the
-    largest value) and in type 3 to 2.5e-6."""
+    transforms give 4e-7 at most in the cases tried, and points crowded at a
+    centre are allowed twice that. The modes at the edge of the box are divided
+    by the kernel's small transform there, which at upsampling 1.25 raises that
+    rounding to 3.2e-5 (3.1e-3 of a single value) and in type 3 to 2.5e-6."""
     if case["call"] == "t3":
         return {"rel": 1e-5}
     if case["sigma"] != 2.0:

@@ -532,6 +532,27 @@ int mn_pad_deconv_fft(int dim, const int64_t n_up[3], const int64_t N[3], int64_
                       int isign, const void *fk, const float *const dec[3], void *work,
                       int64_t work_bytes, void *grid, mn_stream_t stream);
 /*
+ * The same two transforms for fine grids of any size 2^a 3^b 5^c
+ * (mn_fftg_supported: axes of at least 4 and, split, up to 2048^2, longer ones than 2048 split into two
+ * passes). ext gives the extents the grid is stored with (NULL: n_up);
+ * ext[d] in [n_up[d], 2 n_up[d]], larger ones in 2D and 3D only and with a
+ * last axis of at most 2048. Type 1 adds the cells at x + n_up[d] < ext[d]
+ * to cell x before it transforms; type 2 stores every cell at all its images
+ * inside the extents. work: mn_fftg_work_bytes(...) bytes. The first use of
+ * an axis length on a device builds a small twiddle table (kept until
+ * mn_fft_cache_clear).
+ * ref: nd.py:374-383, nd.py:416-435, nd.py:878-906.
+ */
+int mn_fftg_supported(int dim, const int64_t n[3]);
+int64_t mn_fftg_work_bytes(int dim, const int64_t n[3], const int64_t N[3], int64_t batch);
+int mn_fftg_crop_deconv(int dim, const int64_t n_up[3], const int64_t N[3], const int64_t ext[3],
+                        int64_t batch, int isign, const void *grid, const float *const dec[3],
+                        void *work, int64_t work_bytes, void *fk, mn_stream_t stream);
+int mn_fftg_pad_deconv(int dim, const int64_t n_up[3], const int64_t N[3], const int64_t ext[3],
+                       int64_t batch, int isign, const void *fk, const float *const dec[3],
+                       void *work, int64_t work_bytes, void *grid, mn_stream_t stream);
+
+/*
  * The same transform in double precision (complex128 data, rocFFT double).
  * The type-3 pipeline runs its inner-grid FFT this way: its target
  * deconvolution 1/phihat(theta) reaches ~1e2 at the band edges and

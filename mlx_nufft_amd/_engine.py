@@ -697,6 +697,38 @@ def pad_deconv_fft(n_up, N, fk, decs, grid, isign, work, batch=1):
                                       L.stream()), "pad_deconv_fft")
 
 
+def fftg_supported(n_up):
+    """True when the general pruned FFT applies (5-smooth fine-grid sizes);
+    MN_FFT=rocfft forces full rocFFT + crop/pad."""
+    if os.environ.get("MN_FFT", "") == "rocfft":
+        return False
+    return bool(L.lib().mn_fftg_supported(len(n_up), L.i64x3(n_up)))
+
+
+def fftg_work_bytes(n_up, N, batch=1):
+    return int(L.lib().mn_fftg_work_bytes(len(N), L.i64x3(n_up), L.i64x3(N), int(batch)))
+
+
+def fftg_crop_deconv(n_up, N, grid, decs, fk, isign, work, batch=1, ext=None):
+    """fk = crop(FFT(grid)) * prod_d dec_d with the general pruned FFT; the
+    grid is stored with extents ext (n_up when None)."""
+    L.check(L.lib().mn_fftg_crop_deconv(len(N), L.i64x3(n_up), L.i64x3(N),
+                                        L.i64x3(n_up if ext is None else ext), int(batch),
+                                        int(isign), L.ptr(grid), L.ptr3(decs), L.ptr(work),
+                                        0 if work is None else work.numel(), L.ptr(fk),
+                                        L.stream()), "fftg_crop_deconv")
+
+
+def fftg_pad_deconv(n_up, N, fk, decs, grid, isign, work, batch=1, ext=None):
+    """grid = FFT(pad(fk * prod_d dec_d)) with the general pruned FFT; the
+    grid is stored with extents ext (n_up when None)."""
+    L.check(L.lib().mn_fftg_pad_deconv(len(N), L.i64x3(n_up), L.i64x3(N),
+                                       L.i64x3(n_up if ext is None else ext), int(batch),
+                                       int(isign), L.ptr(fk), L.ptr3(decs), L.ptr(work),
+                                       0 if work is None else work.numel(), L.ptr(grid),
+                                       L.stream()), "fftg_pad_deconv")
+
+
 def pad_deconv_c128(n_up, N, fk128, decs64, grid128, batch=1):
     """grid128 = pad(fk128 * prod_d dec_d), complex128 with fp64 factors."""
     L.check(L.lib().mn_pad_deconv_c128(len(N), L.i64x3(n_up), L.i64x3(N), int(batch), L.ptr(fk128),

@@ -128,6 +128,12 @@ _SIGS = [
                                    c_vp, c_vp]),
     ("mn_pad_deconv_fft", c_int, [c_int, I64x3, I64x3, c_int64, c_int, c_vp, VP3, c_vp, c_int64,
                                   c_vp, c_vp]),
+    ("mn_fftg_supported", c_int, [c_int, I64x3]),
+    ("mn_fftg_work_bytes", c_int64, [c_int, I64x3, I64x3, c_int64]),
+    ("mn_fftg_crop_deconv", c_int, [c_int, I64x3, I64x3, I64x3, c_int64, c_int, c_vp, VP3, c_vp,
+                                    c_int64, c_vp, c_vp]),
+    ("mn_fftg_pad_deconv", c_int, [c_int, I64x3, I64x3, I64x3, c_int64, c_int, c_vp, VP3, c_vp,
+                                   c_int64, c_vp, c_vp]),
     ("mn_fill_zero", c_int, [c_vp, c_int64, c_vp]),
 ]
 

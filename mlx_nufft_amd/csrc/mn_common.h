@@ -64,6 +64,8 @@ int max_lds_per_block();
 
 // Releases the cached twiddle tables of the fp64 line FFTs (mn_fftl.hip).
 void fftl_cache_clear();
+// ... and of the general pruned FFTs (mn_fftg.hip).
+void fftg_cache_clear();
 
 // Zero device memory with a fill kernel (usable under graph capture).
 int fill_zero(void *ptr, int64_t bytes, hipStream_t s);

@@ -170,6 +170,7 @@ int mn_fft_cache_clear(void) {
     for (auto &kv : g_plans) destroy_plan(kv.second);
     g_plans.clear();
     fftl_cache_clear();
+    fftg_cache_clear();
     return MN_OK;
 }
 

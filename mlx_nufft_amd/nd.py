@@ -128,7 +128,8 @@ class _PointsND:
             self.decs.append(1.0 / kernel_ft(2.0 * PI * k / self.n_up[d], self.beta, self.w))
         self.dev_dec = [torch.from_numpy(v.astype(np.float32)).to(self.device) for v in self.decs]
         self._grid = None
-        self._pruned = E.fftp_supported(self.n_up)
+        self._pow2 = E.fftp_supported(self.n_up)
+        self._pruned = self._pow2 or E.fftg_supported(self.n_up)
         self._work = None
 
     # the z-sweep point state is built in the spread's key order unless set
@@ -210,7 +211,7 @@ class _PointsND:
 
     def _fft_work(self, batch=1):
         """Work buffer of the pruned FFT (intermediate per-axis arrays)."""
-        nbytes = E.fftp_work_bytes(self.n_up, self.N, batch)
+        nbytes = (E.fftp_work_bytes if self._pow2 else E.fftg_work_bytes)(self.n_up, self.N, batch)
         if nbytes <= 0:
             return None
         if self._work is None or self._work.numel() < nbytes:
@@ -304,9 +305,10 @@ class Type1PlanND(_PointsND):
 
     def _fft_crop(self, grid, fk, tm, batch):
         if self._pruned:
+            crop = E.fft_crop_deconv if self._pow2 else E.fftg_crop_deconv
             with tm("fft"):
-                E.fft_crop_deconv(self.n_up, self.N, grid, self.dev_dec, fk, self.isign,
-                                  self._fft_work(batch), batch=batch)
+                crop(self.n_up, self.N, grid, self.dev_dec, fk, self.isign,
+                     self._fft_work(batch), batch=batch)
             return
         with tm("fft"):
             E.fft(grid, self.n_up, self.isign, batch=batch)
@@ -431,9 +433,9 @@ class Type2PlanND(_PointsND):
         out = torch.empty(self.P, dtype=torch.complex64, device=self.device)
         tm = self._timer()
         if self._pruned:
+            pad = E.pad_deconv_fft if self._pow2 else E.fftg_pad_deconv
             with tm("fft"):
-                E.pad_deconv_fft(self.n_up, self.N, fd, self.dev_dec, grid, self.isign,
-                                 self._fft_work(1))
+                pad(self.n_up, self.N, fd, self.dev_dec, grid, self.isign, self._fft_work(1))
         else:
             with tm("deconv"):
                 E.pad_deconv(self.n_up, self.N, fd, self.dev_dec, grid)

@@ -91,6 +91,41 @@ def make_bins(dim, w, n_up, m=None, cell_bytes=SPREAD_CELL_BYTES, npts=None):
     return L.Bins.make(dim, w, list(n_up), m)
 
 
+def spread_bins(dim, w, n_up, P):
+    """Bins of the type-1 tile spread for about P points. Bins of 17 - w cells
+    give padded tiles of at most 16 cells per dim, which are accumulated on the
+    matrix cores; their work per point hardly depends on w, where LDS atomics
+    cost w^dim, but smaller tiles flush more halo cells. So the matrix cores
+    take 3D from w = 5 (us, LDS / matrix cores: 1e6 points on 200 x 180 x 160,
+    w = 4: 191 / 219; on 240^3 7e3 to 1.4e6 points, w = 5: 110 / 57 to
+    401 / 373, w = 7: 178 / 69 to 798 / 563, w = 12: 763 / 135 to 7928 / 3576)
+    and 2D from w = 5 where the points fill the grid (2000^2, w = 6: 0.3
+    points per cell 90 / 101, 0.6 143 / 101, 2.4 506 / 281; w = 12: 0.3
+    272 / 387, 0.6 505 / 408); wider 2D kernels leave bins of 4 cells or fewer
+    and need more. MN_BIN_M overrides the bins."""
+    if dim == 1 or w <= 4 or os.environ.get("MN_BIN_M"):
+        return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
+    if dim == 2:
+        full = 0.4 if w <= 12 else 1.0
+        if w > 14 or P < full * float(n_up[0]) * float(n_up[1]):
+            return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
+    return make_bins(dim, w, n_up, m=[max(1, min(17 - w, int(k))) for k in n_up])
+
+
+def spread_msub(bins, P):
+    """Points per subproblem of the type-1 tile spread: MSUB, but in steps of
+    the matrix-core kernels' 64-point batches fewer where MSUB would leave the
+    chip idle (2D tiles take one wave, 3D ones four): 1e4 points on
+    18 x 24 x 30, w = 7, take 27 us instead of 100, 5e5 on 66 x 74 36 instead
+    of 50; 5e5 points on 144 x 128 x 125 already fill it (more, smaller ones
+    flush more tiles: 585 against 527 us for 4 vectors). The LDS kernels keep
+    MSUB (1e5 points in 1D: 17 us, 19 to 25 with fewer)."""
+    dim, w = bins.dim, bins.w
+    if dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
+        return MSUB
+    return max(64, min(MSUB, (P // (2048 if dim == 2 else 512) + 63) // 64 * 64))
+
+
 def key_bits(bins):
     return max(1, int(bins.nbins - 1).bit_length())
 
@@ -415,7 +450,7 @@ class GroupSplit:
             if pts.kind == "tiles":
                 sub = _Subset("tiles", pts.bins, e - s, perm=c[1][s:e], skey=c[0][s:e], frs=frs,
                               i1s=[r[s:e] for r in c[2 + dim:2 + 2 * dim]])
-                sub.info, sub.nsub = build_subproblems(pts.bins, sub.skey)
+                sub.info, sub.nsub = build_subproblems(pts.bins, sub.skey, spread_msub(pts.bins, sub.P))
                 yield g, sub
                 continue
             if self._startbuf is None:

@@ -11,9 +11,9 @@
 // to the periodic fine grid with global atomics (fp32, or fp64 into a
 // complex128 grid), one component per lane so that an instruction's lanes
 // hit adjacent addresses, skipping components that stayed zero. Workgroups
-// are remapped so each XCD walks a contiguous run of bins. 3D fp64 tiles of
+// are remapped so each XCD walks a contiguous run of bins. 2D and 3D tiles of
 // at most 16 cells per dim are accumulated on the matrix cores instead
-// (k_spread_tile_mfma).
+// (k_spread_tile2_mfma, k_spread_tile_mfma), also in fp64.
 // ref: nd.py:492-579 (OD spread), nd.py:683-742 (batched), gpu_t3.py:565-591.
 #include "mn_common.h"
 
@@ -258,13 +258,21 @@ __global__ __launch_bounds__(256) void k_spread_tiled(Geom g, float bl2e, float 
 typedef double mn_v4d __attribute__((ext_vector_type(4)));
 constexpr int MN_SUB_MAX_ORDER = 1024;  // points per subproblem the x-order takes
 
-template <int W>
+//
+// Real is the grid's component type: double for type-3 sources, float for the
+// types 1 and 2, whose vectors blockIdx.y walks (strides cstride and gstride).
+// With a float grid, 2e6 points and w = 7 on 270 x 240 x 180 take 0.56 ms
+// (LDS atomics: 1.11), radial points 0.83 (5.85), 1e6 points and w = 9 on
+// 160^3 0.39 (1.10).
+template <int W, typename Real>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
 k_spread_tile_mfma(Geom g, float bl2e, float inv_hw, int64_t nsub,
                    const int32_t *__restrict__ info, const uint32_t *__restrict__ perm, CI3s i1s,
-                   CF3s frs, const float2 *__restrict__ c, const float2 *__restrict__ pre,
-                   double *__restrict__ grid) {
+                   CF3s frs, const float2 *__restrict__ c, int64_t cstride,
+                   const float2 *__restrict__ pre, Real *__restrict__ grid, int64_t gstride) {
     static_assert(W <= 16, "the footprint must fit a 16-cell tile");
+    c += blockIdx.y * cstride;
+    grid += blockIdx.y * gstride;
     constexpr int NWV = 4;        // waves
     constexpr int NT = 64 * NWV;  // threads
     constexpr int PX = 4 * NWV;   // x planes
@@ -451,9 +459,106 @@ k_spread_tile_mfma(Geom g, float bl2e, float inv_hw, int64_t nsub,
                     const int g2 = wrap_tile(o2 + z, g.n[2]);
                     unsafeAtomicAdd(grid + 2 * (((int64_t)g0 * g.n[1] + g1) * g.n[2] + g2) +
                                         (lane & 1),
-                                    v);
+                                    (Real)v);
                 }
             }
+        }
+    }
+}
+
+// 2D tile spread on the matrix cores, for padded tiles of at most 16 x 16
+// cells (bins of 17 - w): one wavefront per subproblem sums its tile as
+// D[x][y] += sum over 4 points k of wx_k(x) (c_k wy_k(y)) with
+// v_mfma_f64_16x16x4f64, one accumulator for the real and one for the
+// imaginary part, products and sums in fp64. Per batch of 64 points a lane
+// per point writes the point's x and y weight rows (zero off the footprint)
+// and strength to LDS; the K-steps form c wy in fp64 from them. Two MFMAs per
+// 4 points, whatever w: the LDS-atomic tiles retire 2 w^2 fp64 atomics per
+// point instead and were bound by them. The flush goes out in lane pairs as
+// in the 3D kernel.
+// 2e6 points and w = 6 on 1250 x 900 take 80 us (LDS atomics on 32 x 32 bins:
+// 130), 8 vectors of 5e5 points and w = 9 on 432^2 0.15 ms (0.67); the fp64
+// MFMAs alone are 26 us of the former, the weights and tables most of the rest.
+template <int W>
+__global__ __launch_bounds__(64) void k_spread_tile2_mfma(
+    Geom g, float bl2e, float inv_hw, int64_t nsub, const int32_t *__restrict__ info,
+    const uint32_t *__restrict__ perm, CI3s i1s, CF3s frs, const float2 *__restrict__ c,
+    int64_t cstride, float *__restrict__ grid, int64_t gstride) {
+    static_assert(W <= 16, "the footprint must fit a 16-cell tile");
+    constexpr int NB = 64;
+    __shared__ __align__(16) float xw[NB][16], yw[NB][16];
+    __shared__ float2 cs[NB];
+    c += blockIdx.y * cstride;
+    grid += blockIdx.y * gstride;
+    const int lane = threadIdx.x;
+    const int64_t sub = xcd_remap(blockIdx.x, nsub);
+    const int bin = info[3 * sub], s0 = info[3 * sub + 1], cnt = info[3 * sub + 2];
+    const int b0 = bin / g.nb[1], b1 = bin - b0 * g.nb[1];
+    mn_v4d are = {0.0, 0.0, 0.0, 0.0}, aim = {0.0, 0.0, 0.0, 0.0};
+    const int i = lane & 15, k = lane >> 4;
+    // the next batch's point is loaded while the current one is swept
+    int ix = 0, iy = 0;
+    float fx = 0.f, fy = 0.f;
+    float2 cv = make_float2(0.f, 0.f);
+    auto load = [&](int bb) __attribute__((always_inline)) {
+        const int64_t j = (int64_t)s0 + min(bb + lane, cnt - 1);
+        ix = i1s.p[0][j];
+        iy = i1s.p[1][j];
+        fx = frs.p[0][j];
+        fy = frs.p[1][j];
+        cv = c[perm[j]];
+    };
+    load(0);
+    for (int bb = 0; bb < cnt; bb += NB) {
+        const int nb = min(NB, cnt - bb);
+        __syncthreads();  // the previous batch's K-steps are done with the tables
+        {
+            const bool valid = lane < nb;
+            int lx = local_cell(ix, W / 2, g.n[0], b0, g.m[0]);
+            int ly = local_cell(iy, W / 2, g.n[1], b1, g.m[1]);
+            lx = lx < 0 ? 0 : lx;  // cannot happen for keys built by setpts
+            ly = ly < 0 ? 0 : ly;
+            float4 *rx = reinterpret_cast<float4 *>(&xw[lane][0]);
+            float4 *ry = reinterpret_cast<float4 *>(&yw[lane][0]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                rx[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+                ry[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            cs[lane] = valid ? cv : make_float2(0.f, 0.f);
+            if (valid) {
+#pragma unroll
+                for (int a = 0; a < W; ++a) {
+                    xw[lane][lx + a] = es_weight_stable((float)a - fx, bl2e, inv_hw);
+                    yw[lane][ly + a] = es_weight_stable((float)a - fy, bl2e, inv_hw);
+                }
+            }
+        }
+        if (bb + NB < cnt) load(bb + NB);
+        __syncthreads();
+        for (int s = 0; s < (nb + 3) >> 2; ++s) {
+            const int pt = 4 * s + k;
+            const double a = (double)xw[pt][i], wy = (double)yw[pt][i];
+            const float2 cp = cs[pt];
+            are = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cp.x * wy, are, 0, 0, 0);
+            aim = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cp.y * wy, aim, 0, 0, 0);
+        }
+    }
+    // lane l holds D[x = 4 r + l / 16][y = l % 16] in entry r
+    const int o0 = b0 * g.m[0] - W / 2, o1 = b1 * g.m[1] - W / 2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int src = 32 * h + (lane >> 1);
+            const double vre = __shfl(are[r], src, 64), vim = __shfl(aim[r], src, 64);
+            const double v = (lane & 1) ? vim : vre;
+            const int y = src & 15, x = 4 * r + (src >> 4);
+            if (x < g.p[0] && y < g.p[1] && v != 0.0)
+                unsafeAtomicAdd(grid + 2 * ((int64_t)wrap_tile(o0 + x, g.n[0]) * g.n[1] +
+                                            wrap_tile(o1 + y, g.n[1])) +
+                                    (lane & 1),
+                                (float)v);
         }
     }
 }
@@ -952,21 +1057,40 @@ struct SpreadLaunch {
         const float inv_hw = (float)(2.0 / W);
         const int64_t T = tile_cells(a.g);
         const bool batch = a.bc > 1 || a.b0 > 0;
+        if (a.nsub == 0) return MN_OK;
+        if constexpr (DIM >= 2 && W <= 16) {
+            // padded tiles of at most 16 cells per dim: the matrix cores
+            const bool small = g.p[0] <= 16 && g.p[1] <= 16 && g.p[2] <= 16;
+            const dim3 nwg((unsigned)a.nsub, (unsigned)a.bc);
+            const float2 *c = a.c + a.b0 * a.P;
+            const int64_t gsz = (int64_t)g.n[0] * g.n[1] * g.n[2];
+            if constexpr (DIM == 3) {
+                if (a.f64 && !batch && small && spread_tile_mfma()) {
+                    k_spread_tile_mfma<W, double><<<nwg, 256, 0, a.s>>>(
+                        g, bl2e, inv_hw, a.nsub, a.info, a.perm, a.i1s, a.frs, c, 0, a.pre,
+                        static_cast<double *>(a.grid), 0);
+                    MN_LAUNCH_CHECK("spread (matrix-core tiles)");
+                    return MN_OK;
+                }
+                if (!a.f64 && small) {
+                    k_spread_tile_mfma<W, float><<<nwg, 256, 0, a.s>>>(
+                        g, bl2e, inv_hw, a.nsub, a.info, a.perm, a.i1s, a.frs, c, a.P, a.pre,
+                        static_cast<float *>(a.grid) + 2 * a.b0 * gsz, 2 * gsz);
+                    MN_LAUNCH_CHECK("spread (matrix-core tiles)");
+                    return MN_OK;
+                }
+            } else if (!a.f64 && !a.pre && small) {
+                k_spread_tile2_mfma<W><<<nwg, 64, 0, a.s>>>(
+                    g, bl2e, inv_hw, a.nsub, a.info, a.perm, a.i1s, a.frs, c, a.P,
+                    static_cast<float *>(a.grid) + 2 * a.b0 * gsz, 2 * gsz);
+                MN_LAUNCH_CHECK("spread (matrix-core tiles)");
+                return MN_OK;
+            }
+        }
         const size_t lds = (size_t)2 * T * sizeof(double) * (batch ? a.bc : 1);
         if (lds > (size_t)max_lds_per_block()) {
             set_error("spread: tile does not fit in LDS; use smaller bins");
             return MN_EINVAL;
-        }
-        if (a.nsub == 0) return MN_OK;
-        if constexpr (DIM == 3 && W <= 16) {
-            if (a.f64 && !batch && g.p[0] <= 16 && g.p[1] <= 16 && g.p[2] <= 16 &&
-                spread_tile_mfma()) {
-                k_spread_tile_mfma<W><<<(unsigned)a.nsub, 256, 0, a.s>>>(
-                    g, bl2e, inv_hw, a.nsub, a.info, a.perm, a.i1s, a.frs, a.c, a.pre,
-                    static_cast<double *>(a.grid));
-                MN_LAUNCH_CHECK("spread (matrix-core tiles)");
-                return MN_OK;
-            }
         }
         auto kern = batch   ? k_spread_tiled<DIM, W, true, false>
                     : a.f64 ? k_spread_tiled<DIM, W, false, true>
@@ -1105,6 +1229,10 @@ int mn_spread_batch(const mn_bins *g, float beta, int64_t P, int64_t nsub,
     const int64_t tile_bytes = 16 * tile_cells(g);
     int64_t per = (max_lds_per_block() / 2) / tile_bytes;
     if (per < 1) per = 1;
+    // tiles on the matrix cores hold one vector each: all of them in one launch
+    bool small = g->dim >= 2;
+    for (int d = 0; d < g->dim; ++d) small = small && g->m[d] + g->w - 1 <= 16;
+    if (small) per = 65535;
     if (per > B) per = B;
     for (int64_t v0 = 0; v0 < B; v0 += per) {
         a.b0 = v0;

@@ -104,6 +104,8 @@ class _PointsND:
         self._stream_interp = self._use_zstream and E.zstream_eligible(self.dim, self.w)
         if self._stream_interp:
             self.bins = E.make_bins(3, self.w, self.n_up, m=E.ZSTREAM_M)
+        elif self._cell_bytes == E.SPREAD_CELL_BYTES:
+            self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
         else:
             self.bins = E.make_bins(self.dim, self.w, self.n_up, cell_bytes=self._cell_bytes)
         self._zsweep = E.zsweep_eligible(self.dim, self.w, self.n_up) and self._zsweep_wanted()
@@ -140,6 +142,10 @@ class _PointsND:
         return self._use_zsweep
 
     # -- point state -------------------------------------------------------
+
+    def _msub(self):
+        """Points per subproblem of the tile kernels."""
+        return E.MSUB
 
     def _coords(self, x):
         x64 = [L.to_dev_f64(v, self.device) for v in x]
@@ -186,7 +192,8 @@ class _PointsND:
             with tm("setpts"):
                 i1, fr, key = E.setpts_t12(self.bins, x64, self.prec == "crit64")
             with tm("sort+tables"):
-                self.pts = E.SortedPoints(self.bins, i1, fr, key, stream=self._stream_interp)
+                self.pts = E.SortedPoints(self.bins, i1, fr, key, stream=self._stream_interp,
+                                          msub=self._msub())
                 del i1, fr, key
         self.sorted = True
         self._od = True
@@ -267,6 +274,9 @@ class Type1PlanND(_PointsND):
         self.spread_method = spread_method
         self._use_zsweep = spread_method != "gm"
         super().__init__(x, n_modes, eps, isign, upsampfac, prec, sort_points)
+
+    def _msub(self):
+        return E.spread_msub(self.bins, self.P)
 
     def _strengths(self, c):
         cd = L.to_dev_c64(c, self.device).reshape(-1)

@@ -294,6 +294,35 @@ int mn_interp_zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zs
                       mn_stream_t stream);
 
 /*
+ * The z-sweep and the z-gather on grids of any size, stored with larger
+ * extents: g->n holds the extents (the sizes mn_zsweep_nkeys accepts), n the
+ * periodic grid, n[d] + w - 1 <= g->n[d]. mn_zsweep_setpts_ext makes the point
+ * words for the spread (gather = 0) or the interpolation (gather = 1), with
+ * every footprint inside the extents, unwrapped; mn_spread_zsweep_ext spreads
+ * B vectors into grids of the extents (the cells at n[d] and above are images
+ * to be added to cell x - n[d], as mn_fftg_crop_deconv does), and
+ * mn_interp_zgather_ext reads such grids with their images filled in
+ * (mn_fftg_pad_deconv). Both evaluate the kernel's exponent without
+ * cancellation. mn_zsweep_maxload writes the largest number of points one
+ * wavefront of a sweep in segments of zseg visits (device int32), which bounds
+ * the sweep's time where points crowd.
+ * ref: nd.py:152-165, nd.py:492-579, nd.py:974-1073.
+ */
+int mn_zsweep_setpts_ext(const mn_bins *g, const int64_t n[3], int gather, int64_t P,
+                         const double *const x[3], int prec64, uint32_t *word,
+                         float *const fr[3], mn_stream_t stream);
+int mn_spread_zsweep_ext(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                         const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                         const float *const frs[3], const void *cs, void *grids,
+                         mn_stream_t stream);
+int mn_interp_zgather_ext(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                          const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                          const float *const frs[3], const void *grids, void *outs,
+                          mn_stream_t stream);
+int mn_zsweep_maxload(const mn_bins *g, int gather, int zseg, const int32_t *zstart,
+                      int32_t *maxload, mn_stream_t stream);
+
+/*
  * Owner-computes 2D spread ("y-sweep"), the fast path for 2D type-1 grids
  * with n0 a multiple of 64 (>= 128), w <= 8 and (n0/64)*n1*2 <= 2^26 keys.
  * Each wavefront owns 64 consecutive x-columns over a y-segment of yseg

@@ -258,12 +258,6 @@ def fill_zero(t):
             "fill_zero")
 
 
-# z-segment (cells) owned by one z-sweep wavefront: each segment also sweeps
-# the chunk below it, and 256 halves that overhead against 128 (measured on
-# MI355X at 512^3: 1.48 -> 1.40 ms, 512 no better)
-ZSEG = 256
-
-
 def zsweep_eligible(dim, w, n_up):
     """True when the owner-computes z-sweep spread applies: 3D, w <= 8, the
     x and y fine-grid sizes multiples of 8 (>= 16) and at most 2^23 sort keys
@@ -276,6 +270,53 @@ def zsweep_eligible(dim, w, n_up):
     return (n_up[0] // 8) * (n_up[1] // 8) * (-(-n_up[2] // 8)) * 16 <= 1 << 23
 
 
+def zsweep_segment(n):
+    """z-segment (cells) per wavefront of a sweep over the grid or extents n:
+    the one that minimises rounds x (zseg + 8), a wave sweeping its segment and
+    the chunk below it and about 2048 waves running at once. Measured, us, spread / z-gather, the chosen length
+    and 256 cells: 5e5 points on 128^3, w = 6 (16) 72 / 40 and 206 / 157, 2e6 on
+    256^3 (128) 168 / 149 and 232 / 251, 3e6 on 384 x 400 x 432, w = 7 (64)
+    423 / 668 and 465 / 740; 512^3 keeps 256."""
+    blocks = (n[0] // 8) * (n[1] // 8)
+
+    def cost(z):
+        return max(1.0, blocks * (-(-n[2] // z)) / 2048.0) * (min(z, n[2]) + 8)
+
+    return min((256, 128, 64, 32, 16, 8), key=cost)
+
+
+def zsweep_extents(dim, w, n_up):
+    """Extents that let the z-sweep (and the z-gather) serve a 3D grid off its
+    blocks: every axis holds the grid and the w - 1 cells footprints reach past
+    it, rounded up to whole blocks and chunks, and the transform folds (or
+    fills) that overhang. None where it does not apply: the sweep's own limits,
+    a transform that cannot take extents, grids the sweep takes as they are."""
+    if dim != 3 or zsweep_eligible(dim, w, n_up) or w > 8 or min(n_up) < 16:
+        return None
+    if not fftg_supported(n_up) or n_up[2] > 2048:
+        return None
+    ext = [-(-(int(n) + w - 1) // 8) * 8 for n in n_up]
+    return ext if zsweep_eligible(dim, w, ext) else None
+
+
+def zsweep_load(pts, gather):
+    """Device int32: the points visited by the most loaded wave of a sweep."""
+    load = torch.empty(1, dtype=torch.int32, device=pts.dev)
+    L.check(L.lib().mn_zsweep_maxload(ctypes.byref(pts.bins), int(gather), pts.zseg,
+                                      L.ptr(pts.zstart), L.ptr(load), L.stream()), "zsweep load")
+    return load
+
+
+def zsweep_balanced(load, w, P, gather, slack=1.0):
+    """Whether a sweep is not held up by crowded points: its time is at least
+    that of its most loaded wave (20 points a us for the spread, 8 for the
+    gather), which should not exceed slack times what the tile kernels, which
+    split crowded bins, take for all points (0.04 w and 0.017 w us per 1000).
+    Reads load back (4 bytes, as the tile path's subproblem count)."""
+    per_us, tile_us = (8.0, 0.017e-3) if gather else (20.0, 0.04e-3)
+    return load.item() / per_us <= slack * (30.0 + tile_us * w * P)
+
+
 class ZSweepPoints:
     """Point state for the z-sweep spread (gather=False, kind "zsweep") or
     the z-gather interpolation (gather=True, kind "zgather"): packed point
@@ -284,9 +325,11 @@ class ZSweepPoints:
     by the x cell of their first tap for the gather), and the key start
     table. Given the previous point set of the same plan (prev) with the
     same P and geometry, its device buffers are reused, so re-pointing
-    allocates nothing; prev's contents are overwritten in stream order."""
+    allocates nothing; prev's contents are overwritten in stream order.
+    ngrid: the periodic grid when bins describe larger extents (then ext is
+    True and every footprint lies inside them)."""
 
-    def __init__(self, bins, x64, prec64, prev=None, gather=False):
+    def __init__(self, bins, x64, prec64, prev=None, gather=False, ngrid=None):
         lib = L.lib()
         dev = x64[0].device
         self.kind = "zgather" if gather else "zsweep"
@@ -304,9 +347,15 @@ class ZSweepPoints:
 
         word = buf("word_in", P, torch.int32)
         fr = buf("fr_in", (3, P), torch.float32)
-        setpts = lib.mn_zgather_setpts if gather else lib.mn_zsweep_setpts
-        L.check(setpts(ctypes.byref(bins), P, L.ptr3(x64), int(bool(prec64)), L.ptr(word),
-                       L.ptr3(_rows(fr, 3)), L.stream()), f"{self.kind} setpts")
+        self.ext = ngrid is not None
+        self.zseg = zsweep_segment([int(bins.n[d]) for d in range(3)])
+        L.check(lib.mn_zsweep_setpts_ext(ctypes.byref(bins), L.i64x3(ngrid), int(gather), P,
+                                         L.ptr3(x64), int(bool(prec64)), L.ptr(word),
+                                         L.ptr3(_rows(fr, 3)), L.stream())
+                if self.ext else
+                (lib.mn_zgather_setpts if gather else lib.mn_zsweep_setpts)(
+                    ctypes.byref(bins), P, L.ptr3(x64), int(bool(prec64)), L.ptr(word),
+                    L.ptr3(_rows(fr, 3)), L.stream()), f"{self.kind} setpts")
         self.frs = buf("frs", (3, P), torch.float32)
         ws_bytes = int(lib.mn_sort_pairs_workspace_bytes(P, 3))
         self.word, self.perm, _ = sort_pairs(
@@ -457,7 +506,7 @@ class GroupSplit:
                 self._startbuf = torch.empty(pts.K + 1, dtype=torch.int32,
                                              device=pts.perm.device)
             sub = _Subset(pts.kind, pts.bins, e - s, perm=c[1][s:e], word=c[0][s:e], frs=frs,
-                          K=pts.K)
+                          K=pts.K, ext=getattr(pts, "ext", False), zseg=getattr(pts, "zseg", 0))
             starts_fn = {"zsweep": lib.mn_zsweep_starts, "ysweep": lib.mn_ysweep_starts,
                          "ymfma": lib.mn_ymfma_starts}[pts.kind]
             L.check(starts_fn(ctypes.byref(pts.bins), sub.P, L.ptr(sub.word),
@@ -545,27 +594,34 @@ def permute_c64(perm, c, out):
             "permute")
 
 
-def spread_zsweep(pts, beta, c, grid, pre=None, zseg=ZSEG, presorted=False):
+def spread_zsweep(pts, beta, c, grid, pre=None, zseg=None, presorted=False):
     """grid = spread(c) with the owner-computes z-sweep (overwrites grid).
     c is in caller order, or in sorted order when presorted."""
-    L.check(L.lib().mn_spread_zsweep(ctypes.byref(pts.bins), float(beta), pts.P, int(zseg),
+    if pts.ext:  # (c may hold more points than a subset pts indexes)
+        _require(pre is None, "spread_zsweep: no prephase on a grid stored with extents")
+        L.check(L.lib().mn_spread_zsweep_ext(
+            ctypes.byref(pts.bins), float(beta), pts.P, 1, int(zseg or pts.zseg),
+            L.ptr(pts.zstart), None if presorted else L.ptr(pts.perm), L.ptr(pts.word),
+            L.ptr3(pts.fr_rows()), L.ptr(c), L.ptr(grid), L.stream()), "spread_zsweep")
+        return
+    L.check(L.lib().mn_spread_zsweep(ctypes.byref(pts.bins), float(beta), pts.P,
+                                     int(zseg or pts.zseg),
                                      L.ptr(pts.zstart), None if presorted else L.ptr(pts.perm),
                                      L.ptr(pts.word), L.ptr3(pts.fr_rows()), L.ptr(c), L.ptr(pre),
                                      L.ptr(grid), L.stream()), "spread_zsweep")
 
 
-def spread_zsweep_batch(pts, beta, cs, grids, zseg=ZSEG, presorted=False):
+def spread_zsweep_batch(pts, beta, cs, grids, zseg=None, presorted=False):
     """grids[b] = spread(cs[b]) for B vectors with the z-sweep, one launch
     with a wave per (block, vector) (overwrites grids)."""
     B = cs.shape[0]
     _require(grids.shape[0] == B and cs.shape[1] == pts.P and cs.is_contiguous()
              and grids.is_contiguous(), "spread_zsweep_batch: cs must be (B, P) and grids "
              "(B, n0, n1, n2), both contiguous")
-    L.check(L.lib().mn_spread_zsweep_batch(ctypes.byref(pts.bins), float(beta), pts.P, B,
-                                           int(zseg), L.ptr(pts.zstart),
-                                           None if presorted else L.ptr(pts.perm),
-                                           L.ptr(pts.word), L.ptr3(pts.fr_rows()), L.ptr(cs),
-                                           L.ptr(grids), L.stream()), "spread_zsweep_batch")
+    fn = L.lib().mn_spread_zsweep_ext if pts.ext else L.lib().mn_spread_zsweep_batch
+    L.check(fn(ctypes.byref(pts.bins), float(beta), pts.P, B, int(zseg or pts.zseg),
+               L.ptr(pts.zstart), None if presorted else L.ptr(pts.perm), L.ptr(pts.word),
+               L.ptr3(pts.fr_rows()), L.ptr(cs), L.ptr(grids), L.stream()), "spread_zsweep_batch")
 
 
 def spread(pts, beta, c, grid, pre=None, accumulate=False):
@@ -656,26 +712,38 @@ def interp_direct_preferred(pts, w, n_up):
 
 
 def zgather_preferred(P, w, n_up):
-    """True when the z-gather interpolation should beat the direct gather for
-    P points on the 3D fine grid n_up: the direct gather reads P w^3 taps,
-    the z-gather (8 + w - 1)^2 columns of 8 new z-cells for every 8x8-column
-    block and z-chunk that holds points (16 after a skipped chunk), expected
-    over uniform points. The factor 5 is the crossover measured between the
-    direct and the staged-tile gathers (interp_direct_preferred)."""
+    """True when the z-gather interpolation should beat the direct and the
+    staged-tile gathers for P points on the 3D fine grid n_up. The direct
+    gather reads P w^3 taps, the z-gather (8 + w - 1)^2 columns of 8 new
+    z-cells for every 8x8-column block and z-chunk that holds points (16 after
+    a skipped chunk), expected over uniform points. On grids within the
+    last-level cache (2^25 cells) it has to halve the traffic several times
+    over (a factor 5, as between the direct and the staged-tile gathers), on
+    larger ones, where every halo cell comes from memory, far less; and up to
+    w = 5 its matrix products, padded to 16 rows, cost as much as the tiles'
+    taps. Measured, us, z-gather / tiles: 384 x 400 x 432, 2e6 points, w = 4
+    341 / 266, w = 5 349 / 420, w = 8 439 / 866; 200 x 192 x 180, 1.4e6, w = 4
+    93 / 67, w = 5 98 / 75, w = 6 104 / 104, w = 8 141 / 235; 1.1e7, w = 5
+    555 / 672. (Below 2^18 points the w <= 5 difference is some us.)"""
     nchunks = (n_up[0] / 8.0) * (n_up[1] / 8.0) * -(-n_up[2] // 8)
     lam = float(P) / nchunks
     busy = nchunks * -np.expm1(-lam)
     staged = (8 + w - 1) ** 2 * 8.0 * busy * (1.0 + np.exp(-lam))
+    cells = float(n_up[0]) * float(n_up[1]) * float(n_up[2])
+    if cells >= 2.0 ** 25:
+        return float(P) * w ** 3 >= 1.5 * staged
+    if w <= 5 and P >= 1 << 18 and (w < 5 or P < 1.2 * cells):
+        return False
     return float(P) * w ** 3 >= 5.0 * staged
 
 
-def interp_zgather(pts, beta, grids, outs, B=1, zseg=ZSEG):
+def interp_zgather(pts, beta, grids, outs, B=1, zseg=None):
     """3D interpolation over the z-sweep point state: B grids (B x n_up)
     into B output vectors of P values in caller order (outs: B x P)."""
-    L.check(L.lib().mn_interp_zgather(ctypes.byref(pts.bins), float(beta), pts.P, int(B),
-                                      int(zseg), L.ptr(pts.zstart), L.ptr(pts.perm),
-                                      L.ptr(pts.word), L.ptr3(pts.fr_rows()), L.ptr(grids),
-                                      L.ptr(outs), L.stream()), "interp_zgather")
+    fn = L.lib().mn_interp_zgather_ext if pts.ext else L.lib().mn_interp_zgather
+    L.check(fn(ctypes.byref(pts.bins), float(beta), pts.P, int(B), int(zseg or pts.zseg),
+               L.ptr(pts.zstart), L.ptr(pts.perm), L.ptr(pts.word), L.ptr3(pts.fr_rows()),
+               L.ptr(grids), L.ptr(outs), L.stream()), "interp_zgather")
 
 
 def interp(pts, beta, grid, out, post=None):

@@ -83,6 +83,13 @@ _SIGS = [
     ("mn_zgather_setpts", c_int, [ctypes.POINTER(Bins), c_int64, VP3, c_int, c_vp, VP3, c_vp]),
     ("mn_interp_zgather", c_int, [ctypes.POINTER(Bins), c_float, c_int64, c_int64, c_int, c_vp,
                                   c_vp, c_vp, VP3, c_vp, c_vp, c_vp]),
+    ("mn_zsweep_setpts_ext", c_int, [ctypes.POINTER(Bins), I64x3, c_int, c_int64, VP3, c_int, c_vp,
+                                     VP3, c_vp]),
+    ("mn_spread_zsweep_ext", c_int, [ctypes.POINTER(Bins), c_float, c_int64, c_int64, c_int, c_vp,
+                                     c_vp, c_vp, VP3, c_vp, c_vp, c_vp]),
+    ("mn_interp_zgather_ext", c_int, [ctypes.POINTER(Bins), c_float, c_int64, c_int64, c_int, c_vp,
+                                      c_vp, c_vp, VP3, c_vp, c_vp, c_vp]),
+    ("mn_zsweep_maxload", c_int, [ctypes.POINTER(Bins), c_int, c_int, c_vp, c_vp, c_vp]),
     ("mn_permute_c64", c_int, [c_int64, c_vp, c_vp, c_vp, c_vp]),
     ("mn_pointmajor_c64", c_int, [c_int64, c_int64, c_vp, c_vp, c_vp]),
     ("mn_ysweep_nkeys", c_int64, [ctypes.POINTER(Bins)]),

@@ -82,16 +82,18 @@ __global__ void k_setpts_t12(int64_t P, D3 x, Geom g, double h0, double h1, doub
 // A thread takes ZP_ITEMS points ZP_THREADS apart (coalesced), their
 // coordinate loads all issued before the arithmetic: with one point per
 // thread the kernel waited on memory latency.
+// n0..n2 is the periodic grid, e1 and e2 the extents along y and z that the
+// blocks and chunks of the key divide (the grid's own sizes, or larger).
 constexpr int ZP_THREADS = 256;
 constexpr int ZP_ITEMS = 4;
 template <bool GATHER>
 __global__ __launch_bounds__(ZP_THREADS) void k_zs_setpts(int64_t P, D3 x, int n0, int n1, int n2,
-                                                          int w, double h0, double h1, double h2,
+                                                          int e1, int e2, int w, double h0, double h1, double h2,
                                                           int prec64, uint32_t *__restrict__ word,
                                                           F3 fro) {
     const int64_t j0 = (int64_t)blockIdx.x * (ZP_THREADS * ZP_ITEMS) + threadIdx.x;
     const double halfw = 0.5 * (double)w;
-    const int nzc = (n2 + kZsChunk - 1) / kZsChunk;
+    const int nzc = (e2 + kZsChunk - 1) / kZsChunk;
     double xv[ZP_ITEMS][3];
 #pragma unroll
     for (int i = 0; i < ZP_ITEMS; ++i) {
@@ -109,9 +111,9 @@ __global__ __launch_bounds__(ZP_THREADS) void k_zs_setpts(int64_t P, D3 x, int n
         cell_t12(xv[i][1], h1, halfw, prec64, iy, fy);
         cell_t12(xv[i][2], h2, halfw, prec64, iz, fz);
         if constexpr (GATHER)
-            word[j] = zg_word(pmod(ix, n0), pmod(iy, n1), pmod(iz, n2), n1, nzc);
+            word[j] = zg_word(pmod(ix, n0), pmod(iy, n1), pmod(iz, n2), e1, nzc);
         else
-            word[j] = zs_word(pmod(ix, n0), pmod(iy, n1), pmod(iz, n2), n1, nzc, w);
+            word[j] = zs_word(pmod(ix, n0), pmod(iy, n1), pmod(iz, n2), e1, nzc, w);
         fro.p[0][j] = fx;
         fro.p[1][j] = fy;
         fro.p[2][j] = fz;
@@ -314,7 +316,7 @@ int mn_setpts_t12(const mn_bins *g, int64_t P, const double *const x[3], int pre
     return MN_OK;
 }
 
-static int zs_setpts(bool gather, const mn_bins *g, int64_t P, const double *const x[3],
+static int zs_setpts(bool gather, const mn_bins *g, const int64_t n[3], int64_t P, const double *const x[3],
                      int prec64, uint32_t *word, float *const fr[3], mn_stream_t stream) {
     clear_error();
     int rc = zsweep_check(g);
@@ -328,23 +330,36 @@ static int zs_setpts(bool gather, const mn_bins *g, int64_t P, const double *con
         MN_REQUIRE(x[d] && fr[d], "zsweep setpts: NULL coordinate/output pointer");
         xs.p[d] = x[d];
         fo.p[d] = fr[d];
-        h[d] = kTwoPi / (double)g->n[d];
+        h[d] = kTwoPi / (double)n[d];
     }
     auto kern = gather ? k_zs_setpts<true> : k_zs_setpts<false>;
     kern<<<blocks_for(P, ZP_THREADS * ZP_ITEMS), ZP_THREADS, 0, as_stream(stream)>>>(
-        P, xs, (int)g->n[0], (int)g->n[1], (int)g->n[2], g->w, h[0], h[1], h[2], prec64, word, fo);
+        P, xs, (int)n[0], (int)n[1], (int)n[2], (int)g->n[1], (int)g->n[2], g->w, h[0], h[1], h[2], prec64, word, fo);
     MN_LAUNCH_CHECK("zsweep_setpts");
     return MN_OK;
 }
 
 int mn_zsweep_setpts(const mn_bins *g, int64_t P, const double *const x[3], int prec64,
                      uint32_t *word, float *const fr[3], mn_stream_t stream) {
-    return zs_setpts(false, g, P, x, prec64, word, fr, stream);
+    return zs_setpts(false, g, g ? g->n : nullptr, P, x, prec64, word, fr, stream);
 }
 
 int mn_zgather_setpts(const mn_bins *g, int64_t P, const double *const x[3], int prec64,
                       uint32_t *word, float *const fr[3], mn_stream_t stream) {
-    return zs_setpts(true, g, P, x, prec64, word, fr, stream);
+    return zs_setpts(true, g, g ? g->n : nullptr, P, x, prec64, word, fr, stream);
+}
+
+int mn_zsweep_setpts_ext(const mn_bins *g, const int64_t n[3], int gather, int64_t P,
+                         const double *const x[3], int prec64, uint32_t *word,
+                         float *const fr[3], mn_stream_t stream) {
+    clear_error();
+    int rc = zsweep_check(g);
+    if (rc) return rc;
+    MN_REQUIRE(n != nullptr, "zsweep setpts: NULL grid size");
+    for (int d = 0; d < 3; ++d)
+        MN_REQUIRE(n[d] >= 1 && n[d] + g->w - 1 <= g->n[d],
+                   "zsweep setpts: the extents must hold the grid and w - 1 cells more");
+    return zs_setpts(gather != 0, g, n, P, x, prec64, word, fr, stream);
 }
 
 int mn_ysweep_setpts(const mn_bins *g, int64_t P, const double *const x[2], int prec64,

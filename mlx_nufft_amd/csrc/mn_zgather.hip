@@ -116,8 +116,12 @@ struct ZgPoint {
     float fx, fy, fz;
 };
 
-template <int W>
-__global__ __launch_bounds__(64) void k_interp_zgather(
+// (held to two waves per SIMD: left to itself the compiler gave w = 7 six
+// registers too many for two, and it took 968 us where w = 8 takes 821, for
+// 1.1e7 points on 200 x 192 x 180; so it takes 915, and 1137 instead of
+// 1411 for 1.3e7 points on 384 x 400 x 432)
+template <int W, bool STABLE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_interp_zgather(
     int n0, int n1, int n2, int nbx, int nby, int nzc, int zseg, int nseg, float bl2e,
     const int32_t *__restrict__ zstart, const uint32_t *__restrict__ perm,
     const uint32_t *__restrict__ word, CF3s frs, const float2 *__restrict__ grid,
@@ -281,12 +285,12 @@ __global__ __launch_bounds__(64) void k_interp_zgather(
 #pragma unroll
             for (int a = 0; a < W; ++a) {
                 const float ca = (float)a * ih;
-                wxc[a * TROW] = zs_es(__builtin_fmaf(-fx, ih, ca), bl2e);
-                const float vy = zs_es(__builtin_fmaf(-fy, ih, ca), bl2e) * kAScale;
+                wxc[a * TROW] = zs_es<STABLE>(__builtin_fmaf(-fx, ih, ca), bl2e);
+                const float vy = zs_es<STABLE>(__builtin_fmaf(-fy, ih, ca), bl2e) * kAScale;
                 const auto hv = __builtin_amdgcn_cvt_pkrtz(vy, 0.f);
                 ar[a] = hv[0];
                 ar[16 + a] = (_Float16)(vy - (float)hv[0]);
-                wzt[((s0 + a) & 15) * TROW + lane] = zs_es(__builtin_fmaf(-fz, ih, ca), bl2e);
+                wzt[((s0 + a) & 15) * TROW + lane] = zs_es<STABLE>(__builtin_fmaf(-fz, ih, ca), bl2e);
             }
         }
     };
@@ -454,6 +458,7 @@ struct GArgs {
     const float2 *grid;
     float2 *out;
     int64_t B, P;
+    bool stable;  // weights by the cancellation-free exponent (zs_es)
     hipStream_t s;
 };
 
@@ -471,9 +476,9 @@ struct GLaunch {
             const float bl2e = (float)(a.beta * 1.4426950408889634);
             const int64_t gs = (int64_t)n0 * n1 * n2;
             const dim3 gridd((unsigned)nw, (unsigned)a.B);
-            k_interp_zgather<W><<<gridd, 64, 0, a.s>>>(n0, n1, n2, nbx, nby, nzc, a.zseg, nseg,
-                                                       bl2e, a.zstart, a.perm, a.word, a.frs,
-                                                       a.grid, gs, a.out, a.P);
+            auto kern = a.stable ? k_interp_zgather<W, true> : k_interp_zgather<W, false>;
+            kern<<<gridd, 64, 0, a.s>>>(n0, n1, n2, nbx, nby, nzc, a.zseg, nseg, bl2e, a.zstart,
+                                        a.perm, a.word, a.frs, a.grid, gs, a.out, a.P);
             MN_LAUNCH_CHECK("interp_zgather");
             return MN_OK;
         }
@@ -487,10 +492,10 @@ using namespace mn;
 
 extern "C" {
 
-int mn_interp_zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
-                      const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
-                      const float *const frs[3], const void *grids, void *outs,
-                      mn_stream_t stream) {
+static int zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                   const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                   const float *const frs[3], const void *grids, void *outs, bool stable,
+                   mn_stream_t stream) {
     clear_error();
     int rc = zsweep_check(g);
     if (rc) return rc;
@@ -513,8 +518,23 @@ int mn_interp_zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zs
     a.out = static_cast<float2 *>(outs);
     a.B = B;
     a.P = P;
+    a.stable = stable;
     a.s = as_stream(stream);
     return select_dim_w<GLaunch>(3, g->w, a);
+}
+
+int mn_interp_zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                      const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                      const float *const frs[3], const void *grids, void *outs,
+                      mn_stream_t stream) {
+    return zgather(g, beta, P, B, zseg, zstart, perm, sorted_word, frs, grids, outs, false, stream);
+}
+
+int mn_interp_zgather_ext(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                          const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                          const float *const frs[3], const void *grids, void *outs,
+                          mn_stream_t stream) {
+    return zgather(g, beta, P, B, zseg, zstart, perm, sorted_word, frs, grids, outs, true, stream);
 }
 
 }  // extern "C"

@@ -299,7 +299,7 @@ __device__ __forceinline__ int masked_max9(int v, uint64_t m) {
 #ifndef ZS_OCC
 #define ZS_OCC 2
 #endif
-template <int W, bool PRE, int VB>
+template <int W, bool PRE, int VB, bool STABLE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ZS_OCC))) void
 k_spread_zsweep(int n0, int n1, int n2, int nbx, int nby, int nzc, int zseg, int nseg,
                 float bl2e, const int32_t *__restrict__ zstart, const uint32_t *__restrict__ perm,
@@ -469,17 +469,17 @@ k_spread_zsweep(int n0, int n1, int n2, int nbx, int nby, int nzc, int zseg, int
             const float zo = lx ? 0.f : (float)HW * ih;
 #pragma unroll
             for (int a = 0; a < W; ++a)
-                ew[0][a] = zs_es(__builtin_fmaf(-p.fx, ih, (float)a * ih), bl2e) * kAxisScale;
+                ew[0][a] = zs_es<STABLE>(__builtin_fmaf(-p.fx, ih, (float)a * ih), bl2e) * kAxisScale;
 #pragma unroll
             for (int a = 0; a < HW; ++a)
-                ew[1][a] = zs_es(__builtin_fmaf(-p.fz, ih, zo + (float)a * ih), bl2e);
+                ew[1][a] = zs_es<STABLE>(__builtin_fmaf(-p.fz, ih, zo + (float)a * ih), bl2e);
         } else {
 #pragma unroll
             for (int a = 0; a < W; ++a) {
                 const float ca = (float)a * ih;
-                ew[0][a] = zs_es(__builtin_fmaf(-p.fx, ih, ca), bl2e) * kAxisScale;
-                ew[1][a] = zs_es(__builtin_fmaf(-p.fy, ih, ca), bl2e) * kAxisScale;
-                ew[2][a] = zs_es(__builtin_fmaf(-p.fz, ih, ca), bl2e);
+                ew[0][a] = zs_es<STABLE>(__builtin_fmaf(-p.fx, ih, ca), bl2e) * kAxisScale;
+                ew[1][a] = zs_es<STABLE>(__builtin_fmaf(-p.fy, ih, ca), bl2e) * kAxisScale;
+                ew[2][a] = zs_es<STABLE>(__builtin_fmaf(-p.fz, ih, ca), bl2e);
             }
         }
     };
@@ -684,6 +684,29 @@ k_spread_zsweep(int n0, int n1, int n2, int nbx, int nby, int nzc, int zseg, int
     while (zb < zend) advance();
 }
 
+// The most points any wave of a sweep over zstart visits: those of its
+// segment's chunks, and for the spread those of the chunk below and the ranges
+// that reach it from the -x, -y and -xy blocks (Ranges::fetch).
+__global__ void k_zs_maxload(int nbx, int nby, int nzc, int sc, int nseg, int gather,
+                             const int32_t *__restrict__ zstart, int32_t *__restrict__ maxload) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int v = 0;
+    if (i < (int64_t)nbx * nby * nseg) {
+        const int seg = (int)(i % nseg), by = (int)(i / nseg % nby), bx = (int)(i / nseg / nby);
+        const int lo = max(0, seg * sc - (gather ? 0 : 1)), hi = min(nzc, (seg + 1) * sc);
+        for (int r = 0; r < (gather ? 1 : 4); ++r) {
+            const int x = (r & 1) ? (bx + nbx - 1) % nbx : bx;
+            const int y = (r & 2) ? (by + nby - 1) % nby : by;
+            const int64_t kb = ((int64_t)x * nby + y) * nzc;
+            const int k0 = (r & 1) ? 3 : 0, k1 = r == 0 ? 16 : (r == 1 ? 15 : 12);
+            for (int c = lo; c < hi; ++c) v += zstart[(kb + c) * 16 + k1] - zstart[(kb + c) * 16 + k0];
+        }
+    }
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) v = max(v, __shfl_xor(v, k, 64));
+    if ((threadIdx.x & 63) == 0 && v > 0) atomicMax(maxload, v);
+}
+
 }  // namespace
 
 int zsweep_check(const mn_bins *g) {
@@ -720,6 +743,7 @@ struct ZArgs {
     float2 *grid;
     int64_t B;  // strength vectors (c: B rows of P, grid: B grids)
     int64_t P;
+    bool stable;  // weights by the cancellation-free exponent (zs_es)
     hipStream_t s;
 };
 
@@ -744,7 +768,9 @@ struct ZLaunch {
             int64_t B1 = a.B;
             if (a.B >= 2 && !a.pre && zsweep_pairs()) {
                 const int64_t np = a.B / 2;
-                k_spread_zsweep<W, false, 2><<<dim3((unsigned)nw, (unsigned)np), 64, 0, a.s>>>(
+                auto k2 = a.stable ? k_spread_zsweep<W, false, 2, true>
+                                   : k_spread_zsweep<W, false, 2, false>;
+                k2<<<dim3((unsigned)nw, (unsigned)np), 64, 0, a.s>>>(
                     n0, n1, n2, nbx, nby, nzc, a.zseg, nseg, bl2e, a.zstart, a.perm, a.word,
                     a.frs, a.c, a.P, nullptr, a.grid, gs);
                 MN_LAUNCH_CHECK("spread_zsweep (vector pairs)");
@@ -754,14 +780,11 @@ struct ZLaunch {
             const float2 *c1 = a.c + (a.B - B1) * a.P;
             float2 *g1 = a.grid + (a.B - B1) * gs;
             const dim3 gridv((unsigned)nw, (unsigned)B1);
-            if (a.pre)
-                k_spread_zsweep<W, true, 1><<<gridv, 64, 0, a.s>>>(
-                    n0, n1, n2, nbx, nby, nzc, a.zseg, nseg, bl2e, a.zstart, a.perm, a.word,
-                    a.frs, c1, a.P, a.pre, g1, gs);
-            else
-                k_spread_zsweep<W, false, 1><<<gridv, 64, 0, a.s>>>(
-                    n0, n1, n2, nbx, nby, nzc, a.zseg, nseg, bl2e, a.zstart, a.perm, a.word,
-                    a.frs, c1, a.P, a.pre, g1, gs);
+            auto k1 = a.stable ? k_spread_zsweep<W, false, 1, true>
+                      : a.pre  ? k_spread_zsweep<W, true, 1, false>
+                               : k_spread_zsweep<W, false, 1, false>;
+            k1<<<gridv, 64, 0, a.s>>>(n0, n1, n2, nbx, nby, nzc, a.zseg, nseg, bl2e, a.zstart,
+                                      a.perm, a.word, a.frs, c1, a.P, a.pre, g1, gs);
             MN_LAUNCH_CHECK("spread_zsweep");
             return MN_OK;
         }
@@ -793,7 +816,7 @@ int mn_zsweep_starts(const mn_bins *g, int64_t P, const uint32_t *sorted_word, i
 static int zsweep_spread(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
                          const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
                          const float *const frs[3], const void *c, const void *pre, void *grid,
-                         mn_stream_t stream) {
+                         bool stable, mn_stream_t stream) {
     clear_error();
     int rc = zsweep_check(g);
     if (rc) return rc;
@@ -817,6 +840,7 @@ static int zsweep_spread(const mn_bins *g, float beta, int64_t P, int64_t B, int
     a.grid = static_cast<float2 *>(grid);
     a.B = B;
     a.P = P;
+    a.stable = stable;
     a.s = as_stream(stream);
     return select_dim_w<ZLaunch>(3, g->w, a);
 }
@@ -826,7 +850,7 @@ int mn_spread_zsweep(const mn_bins *g, float beta, int64_t P, int zseg, const in
                      const float *const frs[3], const void *c, const void *pre, void *grid,
                      mn_stream_t stream) {
     return zsweep_spread(g, beta, P, 1, zseg, zstart, perm, sorted_word, frs, c, pre, grid,
-                         stream);
+                         false, stream);
 }
 
 int mn_spread_zsweep_batch(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
@@ -834,7 +858,34 @@ int mn_spread_zsweep_batch(const mn_bins *g, float beta, int64_t P, int64_t B, i
                            const uint32_t *sorted_word, const float *const frs[3],
                            const void *cs, void *grids, mn_stream_t stream) {
     return zsweep_spread(g, beta, P, B, zseg, zstart, perm, sorted_word, frs, cs, nullptr, grids,
-                         stream);
+                         false, stream);
+}
+
+int mn_spread_zsweep_ext(const mn_bins *g, float beta, int64_t P, int64_t B, int zseg,
+                         const int32_t *zstart, const uint32_t *perm, const uint32_t *sorted_word,
+                         const float *const frs[3], const void *cs, void *grids,
+                         mn_stream_t stream) {
+    return zsweep_spread(g, beta, P, B, zseg, zstart, perm, sorted_word, frs, cs, nullptr, grids,
+                         true, stream);
+}
+
+int mn_zsweep_maxload(const mn_bins *g, int gather, int zseg, const int32_t *zstart,
+                      int32_t *maxload, mn_stream_t stream) {
+    clear_error();
+    int rc = zsweep_check(g);
+    if (rc) return rc;
+    MN_REQUIRE(zseg >= ZC && zseg % ZC == 0, "zsweep load: zseg must be a positive multiple of 8");
+    MN_REQUIRE(zstart && maxload, "zsweep load: NULL pointer");
+    hipStream_t s = as_stream(stream);
+    rc = fill_zero(maxload, 4, s);
+    if (rc) return rc;
+    const int nbx = (int)(g->n[0] / ZB), nby = (int)(g->n[1] / ZB);
+    const int nzc = (int)((g->n[2] + ZC - 1) / ZC), sc = zseg / ZC, nseg = (nzc + sc - 1) / sc;
+    const int64_t nw = (int64_t)nbx * nby * nseg;
+    k_zs_maxload<<<(unsigned)((nw + 255) / 256), 256, 0, s>>>(nbx, nby, nzc, sc, nseg, gather,
+                                                              zstart, maxload);
+    MN_LAUNCH_CHECK("zsweep load");
+    return MN_OK;
 }
 
 }  // extern "C"

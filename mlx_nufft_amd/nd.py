@@ -109,8 +109,13 @@ class _PointsND:
         else:
             self.bins = E.make_bins(self.dim, self.w, self.n_up, cell_bytes=self._cell_bytes)
         self._zsweep = E.zsweep_eligible(self.dim, self.w, self.n_up) and self._zsweep_wanted()
-        if self._zsweep:
-            self._zbins = E.make_bins(3, self.w, self.n_up, m=(8, 8, 1))
+        # grids off the sweep's blocks are stored with larger extents, at the
+        # upsampling whose deconvolution does not magnify the sweep's rounding
+        self._ext = None
+        if not self._zsweep and self.sigma >= 2.0 and self._zsweep_wanted():
+            self._ext = E.zsweep_extents(self.dim, self.w, self.n_up)
+        if self._zsweep or self._ext:
+            self._zbins = E.make_bins(3, self.w, self._ext or self.n_up, m=(8, 8, 1))
         # 2D: the y-window MFMA sweep where its geometry applies, else the
         # VALU y-sweep
         self._ymfma = self._use_zsweep and E.ymfma_eligible(self.dim, self.w, self.n_up)
@@ -118,7 +123,7 @@ class _PointsND:
                                              E.ysweep_eligible(self.dim, self.w, self.n_up))
         if self._ysweep:
             self._ybins = E.make_bins(2, self.w, self.n_up, m=(16 if self._ymfma else 64, 1))
-        self._set_points(x64)
+        load = self._set_points(x64, defer=True)
 
         # Mode deconvolution 1/phihat(2 pi k / n_up) on the uncentred fine grid
         # (points folded into [0, 2pi), so no (-1)^k factor). rocFFT's backward
@@ -133,6 +138,10 @@ class _PointsND:
         self._pow2 = E.fftp_supported(self.n_up)
         self._pruned = self._pow2 or E.fftg_supported(self.n_up)
         self._work = None
+        # the host work above has run beside the sort; now look at its result
+        if load is not None and not self._uncrowded(load):
+            self.pts = None
+            self._set_points(x64, tiles=True)
 
     # the z-sweep point state is built in the spread's key order unless set
     _zgather_points = False
@@ -170,17 +179,18 @@ class _PointsND:
         self.i1 = [v.cpu().numpy() for v in i1]
         self.fr = [v.cpu().numpy() for v in fr]
 
-    def _set_points(self, x64):
+    def _set_points(self, x64, defer=False, tiles=False):
+        """Build the point state. Where the sweep has to be looked at for
+        crowding and defer is set, the load is returned for the
+        caller to look at once it has time; tiles builds the tiles' state."""
         tm = self._timer()
-        if self._zsweep:
-            with tm("setpts+sort+tables"):
-                prev = getattr(self, "pts", None)
-                gather = self._zgather_points
-                kind = "zgather" if gather else "zsweep"
-                same = isinstance(prev, E.ZSweepPoints) and prev.kind == kind
-                self.pts = E.ZSweepPoints(self._zbins, x64, self.prec == "crit64",
-                                          prev=prev if same else None, gather=gather)
-                del prev
+        load = None
+        sweep = (self._zsweep or self._ext) and not tiles
+        if sweep:
+            load = self._set_sweep_points(x64, tm)
+            if load is not None and not defer and not self._uncrowded(load):
+                self.pts = None
+                return self._set_points(x64, tiles=True)
         elif self._ysweep:
             with tm("setpts+sort+tables"):
                 prev = getattr(self, "pts", None)
@@ -199,6 +209,42 @@ class _PointsND:
         self._od = True
         self._finish_profile(tm, "setpts")
         self.last_setpts_profile = dict(self.last_profile) if self.profile else {}
+        return load
+
+    # whether the points of the last set held the sweep up (None: no set yet)
+    _crowded = None
+
+    def _set_sweep_points(self, x64, tm):
+        """Point state of the z-sweep or z-gather. Returns its load where the
+        points may hold the sweep up, else None: every set on grids stored
+        with extents; on the sweep's own grids, where re-pointing reads nothing
+        back and results do not depend on the order of atomics, the first set
+        of 2^18 points or more, and further ones while they are crowded."""
+        with tm("setpts+sort+tables"):
+            prev = getattr(self, "pts", None)
+            gather = self._zgather_points
+            kind = "zgather" if gather else "zsweep"
+            same = isinstance(prev, E.ZSweepPoints) and prev.kind == kind
+            self.pts = E.ZSweepPoints(self._zbins, x64, self.prec == "crit64",
+                                      prev=prev if same else None, gather=gather,
+                                      ngrid=self.n_up if self._ext else None)
+            if self._ext or (self._crowded is not False and self.pts.P >= 1 << 18):
+                return E.zsweep_load(self.pts, gather)
+        if self._crowded is None:
+            self._crowded = False
+        return None
+
+    def _uncrowded(self, load):
+        """Whether the sweep keeps the points. Its own grids are left only at
+        three times the tiles' time (radial points on 200 x 192 x 180, 1e6,
+        w = 6: 2.7 ms by the sweep, 0.46 by the tiles)."""
+        self._crowded = not E.zsweep_balanced(load, self.w, self.P, self._zgather_points,
+                                              1.0 if self._ext else 3.0)
+        return not self._crowded
+
+    def _store(self):
+        """Extents the fine grid is stored with (None: n_up) for these points."""
+        return self._ext if getattr(self.pts, "ext", False) else None
 
     @property
     def mx_perm(self):
@@ -210,7 +256,7 @@ class _PointsND:
         return self.pts.perm.cpu().numpy().astype(np.intp)
 
     def _fine_grid(self, batch=1):
-        shape = (batch, *self.n_up)
+        shape = (batch, *(self._store() or self.n_up))
         if self._grid is None or tuple(self._grid.shape) != shape:
             self._grid = None
             self._grid = torch.empty(shape, dtype=torch.complex64, device=self.device)
@@ -315,10 +361,13 @@ class Type1PlanND(_PointsND):
 
     def _fft_crop(self, grid, fk, tm, batch):
         if self._pruned:
-            crop = E.fft_crop_deconv if self._pow2 else E.fftg_crop_deconv
             with tm("fft"):
-                crop(self.n_up, self.N, grid, self.dev_dec, fk, self.isign,
-                     self._fft_work(batch), batch=batch)
+                if self._pow2:
+                    E.fft_crop_deconv(self.n_up, self.N, grid, self.dev_dec, fk, self.isign,
+                                      self._fft_work(batch), batch=batch)
+                else:
+                    E.fftg_crop_deconv(self.n_up, self.N, grid, self.dev_dec, fk, self.isign,
+                                       self._fft_work(batch), batch=batch, ext=self._store())
             return
         with tm("fft"):
             E.fft(grid, self.n_up, self.isign, batch=batch)
@@ -443,9 +492,13 @@ class Type2PlanND(_PointsND):
         out = torch.empty(self.P, dtype=torch.complex64, device=self.device)
         tm = self._timer()
         if self._pruned:
-            pad = E.pad_deconv_fft if self._pow2 else E.fftg_pad_deconv
             with tm("fft"):
-                pad(self.n_up, self.N, fd, self.dev_dec, grid, self.isign, self._fft_work(1))
+                if self._pow2:
+                    E.pad_deconv_fft(self.n_up, self.N, fd, self.dev_dec, grid, self.isign,
+                                     self._fft_work(1))
+                else:
+                    E.fftg_pad_deconv(self.n_up, self.N, fd, self.dev_dec, grid, self.isign,
+                                      self._fft_work(1), ext=self._store())
         else:
             with tm("deconv"):
                 E.pad_deconv(self.n_up, self.N, fd, self.dev_dec, grid)

@@ -467,6 +467,16 @@ int mn_interp(const mn_bins *g, float beta, int64_t P, int64_t nsub,
               const void *grid, const void *post, void *out, mn_stream_t stream);
 
 /*
+ * Mode deconvolution factors of up to three dims, back to back in dec (device,
+ * sum of N[d] floats): 1 / phihat(2 pi k / n_up[d]), k = i - N[d]/2, with
+ * phihat(xi) = 2 sum_q fq[q] cos(xi dq[q]) in fp64 over nquad <= 128 nodes
+ * (host arrays).
+ * ref: nd.py:136-149, sizing.py:74-85.
+ */
+int mn_kernel_dec(int dim, const int64_t N[3], const int64_t n_up[3], const double *dq,
+                  const double *fq, int nquad, float *dec, mn_stream_t stream);
+
+/*
  * Mode shuffle + deconvolution, type 1: for a batch of grids (n_up) and
  * mode boxes (N, modeord=0, k_d in [-(N_d/2), N_d - N_d/2)):
  * fk[b][m] = grid[b][(m - N/2) mod n_up] * prod_d dec_d[m_d].

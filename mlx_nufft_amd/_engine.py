@@ -551,17 +551,20 @@ def spread_ysweep(pts, beta, cs, grids):
                                      L.ptr(cs), L.ptr(grids), L.stream()), "spread_ysweep")
 
 
-def ymfma_segment(n_up, B):
-    """y-segment per wavefront of the y-window MFMA sweep: the longest power
-    of two (<= 256, >= 32) that still gives at least 4096 wavefronts (each
-    segment also sweeps the chunk below it)."""
-    vb = ysweep_vectors_per_wave(B)
-    groups = -(-B // vb)
-    nbx = n_up[0] // 16
-    yseg = 256
-    while yseg > 32 and nbx * (-(-n_up[1] // yseg)) * groups < 4096:
-        yseg //= 2
-    return yseg
+def ymfma_segment(n_up):
+    """y-segment per wavefront of the y-window MFMA sweep: the one (8 to 256
+    cells) that minimises rounds x (yseg + 8), as zsweep_segment, for one wave
+    per block (up to 8 vectors), so that a batch sums as its vectors do alone.
+    Measured, us,
+    the chosen length and the 32 cells that used to be the least: 1e5 points on
+    256^2, w = 7 (8) 21 and 35, 8 vectors 61 and 117; 1e6 on 512^2 (16) 53 and
+    74; 1e7 on 2048^2, 8 vectors (128) 935, 969 at 64."""
+    blocks = n_up[0] // 16
+
+    def cost(y):
+        return max(1.0, blocks * (-(-n_up[1] // y)) / 2048.0) * (min(y, n_up[1]) + 8)
+
+    return min((256, 128, 64, 32, 16, 8), key=cost)
 
 
 def spread_ymfma(pts, beta, cs, grids):
@@ -583,7 +586,7 @@ def spread_ymfma(pts, beta, cs, grids):
         cs = ct
         pm = 1
     L.check(L.lib().mn_spread_ymfma(ctypes.byref(pts.bins), float(beta), pts.P, B,
-                                    ymfma_segment(n_up, B), L.ptr(pts.ystart), L.ptr(pts.perm),
+                                    ymfma_segment(n_up), L.ptr(pts.ystart), L.ptr(pts.perm),
                                     L.ptr(pts.word), V2(pts.frs[0].data_ptr(), pts.frs[1].data_ptr()),
                                     L.ptr(cs), pm, L.ptr(grids), L.stream()), "spread_ymfma")
 
@@ -758,6 +761,16 @@ def interp(pts, beta, grid, out, post=None):
                               L.ptr(pts.info), L.ptr(pts.perm), L.ptr3(pts.i1_rows()),
                               L.ptr3(pts.fr_rows()), L.ptr(grid), L.ptr(post), L.ptr(out),
                               L.stream()), "interp")
+
+
+def kernel_dec(N, n_up, quad, device):
+    """fp32 mode deconvolution factors per dim, 1 / phihat(2 pi k / n_up[d]);
+    quad: the kernel's quadrature (nodes, weights)."""
+    dq, fq = quad
+    out = torch.empty(sum(N), dtype=torch.float32, device=device)
+    L.check(L.lib().mn_kernel_dec(len(N), L.i64x3(N), L.i64x3(n_up), dq.ctypes.data,
+                                  fq.ctypes.data, len(dq), L.ptr(out), L.stream()), "kernel_dec")
+    return list(out.split([int(n) for n in N]))
 
 
 def crop_deconv(n_up, N, grid, decs, fk, batch=1):

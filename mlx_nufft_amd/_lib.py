@@ -113,6 +113,7 @@ _SIGS = [
                                  c_vp, c_vp]),
     ("mn_interp_zstream", c_int, [ctypes.POINTER(Bins), c_float, c_int64, c_vp, c_vp, VP3, VP3,
                                   c_vp, c_vp, c_vp, c_vp]),
+    ("mn_kernel_dec", c_int, [c_int, I64x3, I64x3, c_vp, c_vp, c_int, c_vp, c_vp]),
     ("mn_crop_deconv", c_int, [c_int, I64x3, I64x3, c_int64, c_vp, VP3, c_vp, c_vp]),
     ("mn_pad_deconv", c_int, [c_int, I64x3, I64x3, c_int64, c_vp, VP3, c_vp, c_vp]),
     ("mn_t3_setpts_src", c_int, [ctypes.POINTER(Bins), c_int64, VP3, D3, D3, D3, D3, c_int, c_int,
@@ -198,8 +199,15 @@ def require(cond, msg):
         raise ValueError(msg)
 
 
+# the current stream's handle without building a torch.cuda.Stream object
+# (9 us for the five lookups of a small plan against 2)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream():
-    return c_vp(torch.cuda.current_stream().cuda_stream)
+    if _raw_stream is None:
+        return c_vp(torch.cuda.current_stream().cuda_stream)
+    return c_vp(_raw_stream(torch.cuda.current_device()))
 
 
 def ptr(t):
@@ -236,6 +244,19 @@ def to_dev_f64(a, dev):
         return t.contiguous()
     arr = np.ascontiguousarray(np.asarray(a, dtype=np.float64).ravel())
     return torch.from_numpy(arr).to(dev)
+
+
+def to_dev_f64_all(arrays, dev):
+    """to_dev_f64 of each array; small host arrays of one length (up to 1 MB in
+    all) go over in one copy, as each costs some 17 us whatever its size."""
+    arrays = list(arrays)
+    if len(arrays) > 1 and not any(isinstance(a, torch.Tensor) for a in arrays):
+        host = [np.asarray(a, dtype=np.float64).ravel() for a in arrays]
+        n = host[0].size
+        if all(h.size == n for h in host) and 0 < n * len(host) <= 1 << 17:
+            return list(torch.from_numpy(np.concatenate(host)).to(dev).view(len(host), n))
+        arrays = host
+    return [to_dev_f64(a, dev) for a in arrays]
 
 
 def to_dev_c64(a, dev):

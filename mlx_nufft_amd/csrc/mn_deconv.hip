@@ -112,6 +112,30 @@ __global__ void k_round_c64(int64_t n, const double2 *__restrict__ in, float2 *_
     }
 }
 
+// Mode deconvolution factors dec_d[i] = 1 / phihat(2 pi k / n_d), k = i -
+// N_d/2, of up to three dims, one thread per factor: phihat(xi) = 2 sum_q
+// fq[q] cos(xi dq[q]) in fp64 over the kernel's quadrature (which rides in the
+// launch arguments), rounded to fp32. On the host the 128 cosines per mode
+// were most of building a plan with many modes (5e5 of them in 1D: @DEC@).
+constexpr int kDecQuad = 128;
+struct DecArgs {
+    double dq[kDecQuad], fq[kDecQuad];
+    int nquad;
+    int64_t end[3];  // running totals of N_d
+    int64_t N[3], n[3];
+};
+
+__global__ __launch_bounds__(256) void k_kernel_dec(DecArgs a, float *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= a.end[2]) return;
+    const int d = i < a.end[0] ? 0 : (i < a.end[1] ? 1 : 2);
+    const int64_t N = a.N[d], k = i - (d ? a.end[d - 1] : 0) - N / 2;
+    const double xi = kTwoPi * (double)k / (double)a.n[d];
+    double s = 0.0;
+    for (int q = 0; q < a.nquad; ++q) s += a.fq[q] * cos(xi * a.dq[q]);
+    out[i] = (float)(1.0 / (2.0 * s));
+}
+
 // Right-align dim-sized shapes into 3 slots; dec pointers follow the dims.
 int align3(int dim, const int64_t *a, const int64_t *b, const float *const dec[3], int A[3],
            int Bv[3], Dec3 *D) {
@@ -143,6 +167,34 @@ unsigned grid_blocks(int64_t total) {
 using namespace mn;
 
 extern "C" {
+
+int mn_kernel_dec(int dim, const int64_t N[3], const int64_t n_up[3], const double *dq,
+                  const double *fq, int nquad, float *dec, mn_stream_t stream) {
+    clear_error();
+    MN_REQUIRE(dim >= 1 && dim <= 3, "kernel_dec: dim must be 1, 2 or 3");
+    MN_REQUIRE(dq && fq && dec, "kernel_dec: NULL pointer");
+    MN_REQUIRE(nquad >= 1 && nquad <= kDecQuad, "kernel_dec: 1 to 128 quadrature nodes");
+    DecArgs a{};
+    for (int q = 0; q < nquad; ++q) {
+        a.dq[q] = dq[q];
+        a.fq[q] = fq[q];
+    }
+    a.nquad = nquad;
+    int64_t tot = 0;
+    for (int d = 0; d < 3; ++d) {
+        if (d < dim) {
+            MN_REQUIRE(N[d] >= 1 && n_up[d] >= N[d] && N[d] < (int64_t(1) << 38),
+                       "kernel_dec: mode count out of range");
+            a.N[d] = N[d];
+            a.n[d] = n_up[d];
+            tot += N[d];
+        }
+        a.end[d] = tot;
+    }
+    k_kernel_dec<<<(unsigned)((tot + 255) / 256), 256, 0, as_stream(stream)>>>(a, dec);
+    MN_LAUNCH_CHECK("kernel_dec");
+    return MN_OK;
+}
 
 int mn_crop_deconv(int dim, const int64_t n_up[3], const int64_t N[3], int64_t batch,
                    const void *grid, const float *const dec[3], void *fk, mn_stream_t stream) {

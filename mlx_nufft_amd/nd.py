@@ -23,7 +23,7 @@ import torch
 
 from . import _engine as E
 from . import _lib as L
-from .sizing import kernel_ft, kernel_params, next235even
+from .sizing import kernel_ft, kernel_params, next235even, quadrature
 
 PI = np.pi
 
@@ -129,16 +129,12 @@ class _PointsND:
         # (points folded into [0, 2pi), so no (-1)^k factor). rocFFT's backward
         # transform is unnormalised, so no prod(n_up) factor is folded in
         # (ref: nd.py:136-149 folds it because its ifft divides by n).
-        self.decs = []
-        for d in range(self.dim):
-            k = np.arange(-(self.N[d] // 2), self.N[d] - self.N[d] // 2, dtype=np.float64)
-            self.decs.append(1.0 / kernel_ft(2.0 * PI * k / self.n_up[d], self.beta, self.w))
-        self.dev_dec = [torch.from_numpy(v.astype(np.float32)).to(self.device) for v in self.decs]
+        self.dev_dec = E.kernel_dec(self.N, self.n_up, quadrature(self.beta, self.w), self.device)
         self._grid = None
         self._pow2 = E.fftp_supported(self.n_up)
         self._pruned = self._pow2 or E.fftg_supported(self.n_up)
         self._work = None
-        # the host work above has run beside the sort; now look at its result
+        # the rest of the plan was queued behind the sort; now look at its result
         if load is not None and not self._uncrowded(load):
             self.pts = None
             self._set_points(x64, tiles=True)
@@ -150,6 +146,12 @@ class _PointsND:
         """Whether the point state should be the z-sweep's (3D, eligible grids)."""
         return self._use_zsweep
 
+    @property
+    def decs(self):
+        """The deconvolution factors per dim in fp64, evaluated on the host."""
+        return [1.0 / kernel_ft(2.0 * PI * np.arange(-(N // 2), N - N // 2, dtype=np.float64) / n,
+                                self.beta, self.w) for N, n in zip(self.N, self.n_up)]
+
     # -- point state -------------------------------------------------------
 
     def _msub(self):
@@ -157,7 +159,7 @@ class _PointsND:
         return E.MSUB
 
     def _coords(self, x):
-        x64 = [L.to_dev_f64(v, self.device) for v in x]
+        x64 = L.to_dev_f64_all(x, self.device)
         P = x64[0].numel()
         if P < 1:
             raise ValueError("at least one nonuniform point is required")
@@ -413,7 +415,7 @@ class Type1PlanND(_PointsND):
             raise ValueError(f"expected {self.dim} coordinate arrays, got {len(x)}")
         if backend not in ("host", "gpu"):
             raise ValueError(f"unknown backend {backend!r}")
-        x64 = [L.to_dev_f64(v, self.device) for v in x]
+        x64 = L.to_dev_f64_all(x, self.device)
         P = x64[0].numel()
         if P < 1 or not all(v.numel() == P for v in x64):
             raise ValueError("coordinate arrays must be non-empty, equal length")

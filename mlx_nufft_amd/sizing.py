@@ -5,6 +5,8 @@ These follow the FINUFFT-family formulas the reference uses
 (ref: mlx_nufft/sizing.py:13-111), so grid sizes and kernel shapes match.
 """
 
+import functools
+
 import numpy as np
 
 PI = np.pi
@@ -72,18 +74,24 @@ def es_kernel(d, beta, w):
 _GL = {}
 
 
+@functools.lru_cache(maxsize=64)
+def _quadrature(beta, w, nquad):
+    if nquad not in _GL:
+        _GL[nquad] = np.polynomial.legendre.leggauss(nquad)
+    t, wt = _GL[nquad]
+    dq = 0.5 * (t + 1.0) * (w / 2.0)
+    fq = wt * (w / 4.0) * es_kernel(dq, beta, w)
+    dq.flags.writeable = fq.flags.writeable = False  # shared by every caller
+    return dq, fq
+
+
 def quadrature(beta, w, nquad=128):
     """Nodes dq on [0, w/2] and weights fq = GL weight * psi(dq) such that
     phihat(xi) = 2 * sum_q fq[q] cos(xi dq[q]) (even kernel).
 
     ref: sizing.py:74-85 (128-point Gauss-Legendre on [0, w/2]).
     """
-    if nquad not in _GL:
-        _GL[nquad] = np.polynomial.legendre.leggauss(nquad)
-    t, wt = _GL[nquad]
-    dq = 0.5 * (t + 1.0) * (w / 2.0)
-    fq = wt * (w / 4.0) * es_kernel(dq, beta, w)
-    return dq, fq
+    return _quadrature(float(beta), int(w), int(nquad))
 
 
 def kernel_ft(xi, beta, w, nquad=128):

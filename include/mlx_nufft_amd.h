@@ -389,6 +389,11 @@ int mn_spread_ymfma(const mn_bins *g, float beta, int64_t P, int64_t B, int yseg
                     const float *const frs[2], const void *c, int point_major, void *grid,
                     mn_stream_t stream);
 
+/* The largest number of points one wavefront of the y-window MFMA sweep in
+ * segments of yseg visits (device int32), as mn_zsweep_maxload. */
+int mn_ymfma_maxload(const mn_bins *g, int yseg, const int32_t *ystart, int32_t *maxload,
+                     mn_stream_t stream);
+
 /*
  * out (P x B, point-major) = the transpose of in (B x P, vector-major), for
  * B complex64 strength vectors of P points: the layout mn_spread_ymfma

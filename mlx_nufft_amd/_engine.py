@@ -299,22 +299,32 @@ def zsweep_extents(dim, w, n_up):
     return ext if zsweep_eligible(dim, w, ext) else None
 
 
-def zsweep_load(pts, gather):
+def sweep_load(pts):
     """Device int32: the points visited by the most loaded wave of a sweep."""
     load = torch.empty(1, dtype=torch.int32, device=pts.dev)
-    L.check(L.lib().mn_zsweep_maxload(ctypes.byref(pts.bins), int(gather), pts.zseg,
-                                      L.ptr(pts.zstart), L.ptr(load), L.stream()), "zsweep load")
+    if pts.kind == "ymfma":
+        yseg = ymfma_segment([int(pts.bins.n[0]), int(pts.bins.n[1])])
+        L.check(L.lib().mn_ymfma_maxload(ctypes.byref(pts.bins), yseg, L.ptr(pts.ystart),
+                                         L.ptr(load), L.stream()), "ymfma load")
+    else:
+        L.check(L.lib().mn_zsweep_maxload(ctypes.byref(pts.bins), int(pts.kind == "zgather"),
+                                          pts.zseg, L.ptr(pts.zstart), L.ptr(load), L.stream()),
+                "zsweep load")
     return load
 
 
-def zsweep_balanced(load, w, P, gather, slack=1.0):
+# points a us of one sweep wave, and us the tile kernels, which split crowded
+# bins, take for 1000 points per unit of w
+_SWEEP_RATES = {"zsweep": (20.0, 0.04), "zgather": (8.0, 0.017), "ymfma": (21.0, 0.012)}
+
+
+def sweep_balanced(load, kind, w, P, slack=1.0):
     """Whether a sweep is not held up by crowded points: its time is at least
-    that of its most loaded wave (20 points a us for the spread, 8 for the
-    gather), which should not exceed slack times what the tile kernels, which
-    split crowded bins, take for all points (0.04 w and 0.017 w us per 1000).
-    Reads load back (4 bytes, as the tile path's subproblem count)."""
-    per_us, tile_us = (8.0, 0.017e-3) if gather else (20.0, 0.04e-3)
-    return load.item() / per_us <= slack * (30.0 + tile_us * w * P)
+    that of its most loaded wave, which should not exceed slack times what the
+    tile kernels take for all points. Reads load back (4 bytes, as the tile
+    path's subproblem count)."""
+    per_us, tile_us = _SWEEP_RATES[kind]
+    return load.item() / per_us <= slack * (30.0 + tile_us * 1e-3 * w * P)
 
 
 class ZSweepPoints:
@@ -549,6 +559,16 @@ def spread_ysweep(pts, beta, cs, grids):
                                      ysweep_segment(n_up, B), L.ptr(pts.ystart), L.ptr(pts.perm),
                                      L.ptr(pts.word), V2(pts.frs[0].data_ptr(), pts.frs[1].data_ptr()),
                                      L.ptr(cs), L.ptr(grids), L.stream()), "spread_ysweep")
+
+
+def tiles_beat_ysweep(bins, w, n_up, P):
+    """True when many points on a grid only the VALU y-sweep fits are better
+    spread by the matrix-core tiles (bins: the tiles'): w = 7, us, sweep /
+    tiles, 2e5 points on 256 x 270 412 / 34, 1e6 on 1024 x 900 194 / 63
+    (radial 2366 / 89), 1e7 on 2048 x 2250 486 / 325. MN_SPREAD=ysweep keeps
+    the sweep."""
+    return (os.environ.get("MN_SPREAD", "") != "ysweep" and P >= 1 << 17
+            and bins.m[0] + w - 1 <= 16)
 
 
 def ymfma_segment(n_up):

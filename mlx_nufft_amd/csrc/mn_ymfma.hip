@@ -553,6 +553,25 @@ __global__ __launch_bounds__(PM_THREADS) void k_pointmajor_c64(int64_t B, int64_
     }
 }
 
+// The most points any wave of a sweep over ystart visits: those of its
+// segment's chunks and of the chunk below, and the reaching ones of the -x
+// block.
+__global__ void k_ym_maxload(int nbx, int nyc, int sc, int nseg, const int32_t *__restrict__ ystart,
+                             int32_t *__restrict__ maxload) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int v = 0;
+    if (i < (int64_t)nbx * nseg) {
+        const int seg = (int)(i % nseg), bx = (int)(i / nseg);
+        const int64_t kb = (int64_t)bx * nyc, km = (int64_t)((bx + nbx - 1) % nbx) * nyc;
+        for (int c = max(0, seg * sc - 1); c < min(nyc, (seg + 1) * sc); ++c)
+            v += ystart[(kb + c) * 2 + 2] - ystart[(kb + c) * 2] + ystart[(km + c) * 2 + 2] -
+                 ystart[(km + c) * 2 + 1];
+    }
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) v = max(v, __shfl_xor(v, k, 64));
+    if ((threadIdx.x & 63) == 0 && v > 0) atomicMax(maxload, v);
+}
+
 }  // namespace
 
 }  // namespace mn
@@ -560,6 +579,24 @@ __global__ __launch_bounds__(PM_THREADS) void k_pointmajor_c64(int64_t B, int64_
 using namespace mn;
 
 extern "C" {
+
+int mn_ymfma_maxload(const mn_bins *g, int yseg, const int32_t *ystart, int32_t *maxload,
+                     mn_stream_t stream) {
+    clear_error();
+    int rc = ymfma_check(g);
+    if (rc) return rc;
+    MN_REQUIRE(yseg >= YC && yseg % YC == 0, "ymfma load: yseg must be a positive multiple of 8");
+    MN_REQUIRE(ystart && maxload, "ymfma load: NULL pointer");
+    hipStream_t s = as_stream(stream);
+    rc = fill_zero(maxload, 4, s);
+    if (rc) return rc;
+    const int nbx = (int)(g->n[0] / XB), nyc = (int)(g->n[1] / YC), sc = yseg / YC;
+    const int nseg = (nyc + sc - 1) / sc;
+    const int64_t nw = (int64_t)nbx * nseg;
+    k_ym_maxload<<<(unsigned)((nw + 255) / 256), 256, 0, s>>>(nbx, nyc, sc, nseg, ystart, maxload);
+    MN_LAUNCH_CHECK("ymfma load");
+    return MN_OK;
+}
 
 int64_t mn_ymfma_nkeys(const mn_bins *g) {
     clear_error();

@@ -121,6 +121,9 @@ class _PointsND:
         self._ymfma = self._use_zsweep and E.ymfma_eligible(self.dim, self.w, self.n_up)
         self._ysweep = self._use_zsweep and (self._ymfma or
                                              E.ysweep_eligible(self.dim, self.w, self.n_up))
+        if self._ysweep and not self._ymfma and E.tiles_beat_ysweep(self.bins, self.w, self.n_up,
+                                                                    self.P):
+            self._ysweep = False
         if self._ysweep:
             self._ybins = E.make_bins(2, self.w, self.n_up, m=(16 if self._ymfma else 64, 1))
         load = self._set_points(x64, defer=True)
@@ -182,24 +185,16 @@ class _PointsND:
         self.fr = [v.cpu().numpy() for v in fr]
 
     def _set_points(self, x64, defer=False, tiles=False):
-        """Build the point state. Where the sweep has to be looked at for
-        crowding and defer is set, the load is returned for the
-        caller to look at once it has time; tiles builds the tiles' state."""
+        """Build the point state. Where a sweep has to be looked at for
+        crowding and defer is set, its load is returned for the caller to look
+        at once it has time; tiles builds the tiles' state."""
         tm = self._timer()
         load = None
-        sweep = (self._zsweep or self._ext) and not tiles
-        if sweep:
+        if (self._zsweep or self._ext or self._ysweep) and not tiles:
             load = self._set_sweep_points(x64, tm)
             if load is not None and not defer and not self._uncrowded(load):
                 self.pts = None
                 return self._set_points(x64, tiles=True)
-        elif self._ysweep:
-            with tm("setpts+sort+tables"):
-                prev = getattr(self, "pts", None)
-                self.pts = E.YSweepPoints(self._ybins, x64, self.prec == "crit64",
-                                          prev=prev if isinstance(prev, E.YSweepPoints) else None,
-                                          mfma=self._ymfma)
-                del prev
         else:
             with tm("setpts"):
                 i1, fr, key = E.setpts_t12(self.bins, x64, self.prec == "crit64")
@@ -217,31 +212,42 @@ class _PointsND:
     _crowded = None
 
     def _set_sweep_points(self, x64, tm):
-        """Point state of the z-sweep or z-gather. Returns its load where the
-        points may hold the sweep up, else None: every set on grids stored
-        with extents; on the sweep's own grids, where re-pointing reads nothing
+        """Point state of a sweep or the z-gather. Returns its load where the
+        points may hold it up, else None: every set on grids stored with
+        extents; on the sweeps' own grids, where re-pointing reads nothing
         back and results do not depend on the order of atomics, the first set
-        of 2^18 points or more, and further ones while they are crowded."""
+        of 2^18 points (2^17 in 2D) or more, and further ones while they are
+        crowded."""
+        prec64 = self.prec == "crit64"
         with tm("setpts+sort+tables"):
             prev = getattr(self, "pts", None)
-            gather = self._zgather_points
-            kind = "zgather" if gather else "zsweep"
-            same = isinstance(prev, E.ZSweepPoints) and prev.kind == kind
-            self.pts = E.ZSweepPoints(self._zbins, x64, self.prec == "crit64",
-                                      prev=prev if same else None, gather=gather,
-                                      ngrid=self.n_up if self._ext else None)
-            if self._ext or (self._crowded is not False and self.pts.P >= 1 << 18):
-                return E.zsweep_load(self.pts, gather)
+            if self._ysweep:
+                self.pts = E.YSweepPoints(self._ybins, x64, prec64,
+                                          prev=prev if isinstance(prev, E.YSweepPoints) else None,
+                                          mfma=self._ymfma)
+            else:
+                kind = "zgather" if self._zgather_points else "zsweep"
+                same = isinstance(prev, E.ZSweepPoints) and prev.kind == kind
+                self.pts = E.ZSweepPoints(self._zbins, x64, prec64, prev=prev if same else None,
+                                          gather=self._zgather_points,
+                                          ngrid=self.n_up if self._ext else None)
+            del prev
+            many = self._ymfma if self._ysweep else True
+            many = many and self.P >= 1 << (17 if self._ysweep else 18)
+            if self._ext or (self._crowded is not False and many):
+                return E.sweep_load(self.pts)
         if self._crowded is None:
             self._crowded = False
         return None
 
     def _uncrowded(self, load):
-        """Whether the sweep keeps the points. Its own grids are left only at
-        three times the tiles' time (radial points on 200 x 192 x 180, 1e6,
-        w = 6: 2.7 ms by the sweep, 0.46 by the tiles)."""
-        self._crowded = not E.zsweep_balanced(load, self.w, self.P, self._zgather_points,
-                                              1.0 if self._ext else 3.0)
+        """Whether the sweep keeps the points. The sweeps' own grids are left
+        only at a few times the tiles' time. Measured, us, sweep / tiles, radial
+        points: 1e6 on 200 x 192 x 180, w = 6, spread 2738 / 460, gather
+        2625 / 135; 2D, w = 7, 1e6 on 1024^2 455 / 90, 5e6 on 2048^2
+        1507 / 282."""
+        slack = 1.0 if self._ext else (2.0 if self._ysweep else 3.0)
+        self._crowded = not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack)
         return not self._crowded
 
     def _store(self):

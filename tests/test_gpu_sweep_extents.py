@@ -117,3 +117,21 @@ def test_crowded_points_on_native_grids(mn):
     assert p.pts.kind == "zsweep"
     ref = mn.Type1PlanND(wide, N, eps=eps, spread_method="gm").execute(c)
     assert np.linalg.norm(p.execute(c) - ref) <= 3e-6 * np.linalg.norm(ref)
+
+
+def test_crowded_points_2d(mn):
+    """The 2D sweep hands crowded sets of 2^17 points or more to the tiles, and
+    grids that only the VALU y-sweep fits go to them when they are dense."""
+    print("case crowded 2d", flush=True)
+    rng = np.random.default_rng(35)
+    M, eps = 1 << 17, 1e-6
+    crowd = tuple(rng.uniform(0.1, 0.2, M) for _ in range(2))
+    wide, c = tuple(rng.uniform(-np.pi, np.pi, M) for _ in range(2)), _cplx(rng, M)
+    p = mn.Type1PlanND(crowd, (128, 128), eps=eps)
+    for x, kind in ((crowd, "tiles"), (wide, "ymfma"), (wide, "ymfma")):
+        p.set_sources(x)
+        assert p.pts.kind == kind
+        ref = mn.Type1PlanND(x, (128, 128), eps=eps, spread_method="gm").execute(c)
+        assert np.linalg.norm(p.execute(c) - ref) <= 3e-6 * np.linalg.norm(ref)
+    q = mn.Type1PlanND(wide, (128, 135), eps=eps)     # 256 x 270
+    assert q.pts.kind == "tiles"

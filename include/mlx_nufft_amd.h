@@ -645,6 +645,17 @@ int mn_fft64_lines(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, cons
                    mn_stream_t stream);
 
 /*
+ * The same pass over a part of its lines and outputs: with part = {r0, r1,
+ * period, q0, q1, c0, c1}, line index a * B + b = q * period + c is transformed
+ * for q in [q0, q1) and c in [c0, c1), and outputs r0 <= r < r1 of it are
+ * stored, at the place they have in the whole array; nothing else of `out` is
+ * written. period divides B, or A when B is 1. part == NULL is the whole pass.
+ */
+int mn_fft64_lines_part(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, const void *in,
+                        const double *dec, void *out, int out_c64, int out_layout,
+                        const int64_t *part, mn_stream_t stream);
+
+/*
  * Batched transpose of complex128 matrices: out[b][c][r] = in[b][r][c] for
  * in (Bt, R, C) and out (Bt, C, R), Bt <= 65535; in and out must not
  * overlap. Between the type-3 line passes it turns a strided axis of long

@@ -9,6 +9,7 @@ width, from the LDS budget of one CDNA4 workgroup.
 
 import contextlib
 import ctypes
+import math
 import os
 
 import numpy as np
@@ -890,11 +891,32 @@ def fft64_lines_supported(n):
 FFT64_LAYOUTS = {"anb": 0, "lines_last": 1, "lines_first": 2}
 
 
-def fft64_lines(A, nin, B, n, isign, src128, dec64, out, layout="anb"):
+def target_cells(n, w, R, margin=1):
+    """[lo, hi) holding every tap of targets within R cells of the middle of an
+    axis of n cells, the whole axis where they would wrap. The length is a
+    multiple of 16 or 8 where that fits, so that strided line passes over the
+    range have tiles of as many lines, and lo one of 8 where that is no longer."""
+    lo = math.floor(0.5 * (n - w) - R) - margin
+    hi = math.ceil(0.5 * (n + w) + R) + margin
+    if lo < 0 or hi > n:
+        return 0, n
+    best = (0, n)
+    for start in (lo - lo % 8, lo):
+        for step in (16, 8):
+            end = start + -(-(hi - start) // step) * step
+            if end <= n and end - start < best[1] - best[0]:
+                best = (start, end)
+                break
+    return best
+
+
+def fft64_lines(A, nin, B, n, isign, src128, dec64, out, layout="anb", keep=None, rows=None):
     """One axis pass of the zero-padding fp64 line FFT: src128 (A, nin, B)
     complex128 -> out (A, n, B) ("anb"), (n, A*B) with the line index fastest
     ("lines_last") or (A*B, n) with each line contiguous ("lines_first"),
-    complex128 or complex64 (by out's dtype)."""
+    complex128 or complex64 (by out's dtype). keep = (r0, r1) stores those
+    outputs of each line only; rows = (period, (q0, q1), (c0, c1)) transforms
+    the lines q * period + c in these ranges only (index a * B + b)."""
     _require(layout in FFT64_LAYOUTS, f"fft64_lines: layout must be one of {tuple(FFT64_LAYOUTS)}")
     c64 = out.dtype == torch.complex64
     _require(src128.dtype == torch.complex128 and src128.numel() >= A * nin * B,
@@ -903,9 +925,14 @@ def fft64_lines(A, nin, B, n, isign, src128, dec64, out, layout="anb"):
              f"fft64_lines: out must be complex64/128 with at least {A * n * B} elements")
     _require(dec64 is None or (dec64.dtype == torch.float64 and dec64.numel() >= nin),
              f"fft64_lines: dec must be float64 with at least {nin} elements")
-    L.check(L.lib().mn_fft64_lines(int(A), int(nin), int(B), int(n), int(isign), L.ptr(src128),
-                                   None if dec64 is None else L.ptr(dec64), L.ptr(out), int(c64),
-                                   FFT64_LAYOUTS[layout], L.stream()), "fft64_lines")
+    part = None
+    if keep is not None or rows is not None:
+        period, q, c = rows or ((B, (0, A), (0, B)) if B > 1 else (A, (0, 1), (0, A)))
+        part = (ctypes.c_int64 * 7)(*(keep or (0, n)), period, *q, *c)
+    L.check(L.lib().mn_fft64_lines_part(int(A), int(nin), int(B), int(n), int(isign),
+                                        L.ptr(src128), None if dec64 is None else L.ptr(dec64),
+                                        L.ptr(out), int(c64), FFT64_LAYOUTS[layout], part,
+                                        L.stream()), "fft64_lines")
 
 
 def transpose_c128(Bt, R, C, src, out):

@@ -130,6 +130,8 @@ _SIGS = [
     ("mn_fft64_lines_supported", c_int, [c_int64]),
     ("mn_fft64_lines", c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_vp, c_vp, c_vp, c_int,
                                c_int, c_vp]),
+    ("mn_fft64_lines_part", c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_vp, c_vp, c_vp,
+                                    c_int, c_int, ctypes.POINTER(c_int64), c_vp]),
     ("mn_transpose_c128", c_int, [c_int64, c_int64, c_int64, c_vp, c_vp, c_vp]),
     ("mn_fftp_supported", c_int, [c_int, I64x3]),
     ("mn_fftp_work_bytes", c_int64, [c_int, I64x3, I64x3, c_int64]),

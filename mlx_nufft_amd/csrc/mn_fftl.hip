@@ -27,6 +27,14 @@
 // Workgroups are remapped so consecutive tiles share an XCD (and its L2)
 // when a tile covers less than a cache line.
 //
+// The passes are bound by the memory they move. Type-3 targets reach the
+// middle 1/sigma of every axis only (plus half a kernel width), so a pass may
+// keep a part of its lines and of their outputs: it transforms lines
+// q * period + r with q and r in given ranges and stores outputs [r0, r0 + nr).
+// Skipped cells are neither written nor read. At 640^3 (486^3 values in,
+// middle 536 kept) the passes move 11.4 instead of 15.1 GB; kept ranges of whole
+// multiples of 16 also give odd lengths tiles of several lines.
+//
 // ref: gpu_t3.py:630-651 (t3pad: pad + mode deconvolution), gpu_t3.py:94-148
 // (fft_axis), gpu_t3.py:697-741 (t3padz: the slab path's fused pad, deconv
 // and z-DFT, which this generalises to every axis).
@@ -54,7 +62,15 @@ struct FlPlan {
     int rad[FL_MAXST];
     int ns[FL_MAXST];         // product of the radices before stage s
     float rns[FL_MAXST];      // 1/ns[s]
+    int r0, nr;               // outputs stored: [r0, r0 + nr)
+    float rnr;                // 1/nr
+    int off, period, kc;      // kept line k is line off + (k / kc) * period + k % kc
 };
+
+__device__ __forceinline__ int fl_line(const FlPlan &p, int k) {
+    const int q = k / p.kc;
+    return p.off + q * p.period + (k - q * p.kc);
+}
 
 // q = x / d for 0 <= x < 2^20 and d >= 1, from a float reciprocal r ~ 1/d:
 // the estimate is off by at most one, fixed by one comparison each way.
@@ -213,8 +229,8 @@ __device__ __forceinline__ void fl_stage(double2 *buf, const double2 *__restrict
 
 // T threads, at most VALS values (ti * n) per tile. With B == 1 the tile's
 // lines are consecutive runs of the input and output; with B > 1, ti divides
-// B, so the tile's lines share a and element m of all of them is ti
-// contiguous values.
+// B or the kept part of it, so the tile's lines share a and element m of all
+// of them is ti contiguous values.
 template <int S, bool C64OUT, int T, int VALS>
 __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ in,
                                                    void *__restrict__ out,
@@ -224,7 +240,8 @@ __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ i
     extern __shared__ double2 fl_buf[];
     const int n = p.n, nin = p.nin, lti = p.lti, ts = p.ts, tid = threadIdx.x;
     const int ti = 1 << lti, lmask = ti - 1;
-    const int li0 = (int)xcd_remap(blockIdx.x, ntiles) << lti;
+    const int k0 = (int)xcd_remap(blockIdx.x, ntiles) << lti;  // first kept line
+    const int li0 = fl_line(p, k0);
     const int half = nin / 2;
     // the zero padding: FFT indices [nin - half, n - half) of every line
     const int gap0 = nin - half;
@@ -239,7 +256,7 @@ __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ i
     double fd[FV];
     if (Bn == 1) {
         const int64_t base = (int64_t)li0 * nin;
-        const int cnt = min(ti, nlines - li0) * nin;
+        const int cnt = min(ti, nlines - k0) * nin;
 #pragma unroll
         for (int i = 0; i < FV; ++i) {
             const int e = min(tid + i * T, cnt - 1);
@@ -295,20 +312,21 @@ __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ i
         else
             reinterpret_cast<double2 *>(out)[o] = v;
     };
+    const int nr = p.nr, r0 = p.r0;
     if (Bo == 1) {
-        const int64_t base = (int64_t)li0 * n;
-        const int cnt = min(ti, nlines - li0) * n;
+        const int64_t base = (int64_t)li0 * n + r0;
+        const int cnt = min(ti, nlines - k0) * nr;
         for (int e = tid; e < cnt; e += T) {
-            const int l = fdiv(e, n, p.rn), r = e - l * n;
-            put(base + e, fl_buf[r * ts + l]);
+            const int l = fdiv(e, nr, p.rnr), r = e - l * nr;
+            put(base + (int64_t)l * n + r, fl_buf[(r0 + r) * ts + l]);
         }
     } else {
         const int a = li0 / Bo, b0 = li0 - a * Bo;
-        const int64_t base = (int64_t)a * n * Bo + b0;
-        const int cnt = min(ti, nlines - li0);
-        for (int e = tid; e < n << lti; e += T) {
+        const int64_t base = ((int64_t)a * n + r0) * Bo + b0;
+        const int cnt = min(ti, nlines - k0);
+        for (int e = tid; e < nr << lti; e += T) {
             const int r = e >> lti, l = e & lmask;
-            if (l < cnt) put(base + (int64_t)r * Bo + l, fl_buf[r * ts + l]);
+            if (l < cnt) put(base + (int64_t)r * Bo + l, fl_buf[(r0 + r) * ts + l]);
         }
     }
 }
@@ -354,7 +372,7 @@ __global__ __launch_bounds__(FLL_THREADS) void k_fft64_long(const double2 *__res
     const int half = nin / 2, gap0 = nin - half;
     double2 nxt[FLL_PT];
     auto load = [&](int line) {
-        const double2 *src = in + (int64_t)line * nin;
+        const double2 *src = in + (int64_t)fl_line(p, line) * nin;
 #pragma unroll
         for (int i = 0; i < FLL_PT; ++i) {
             const int e = tid + i * FLL_THREADS;
@@ -388,8 +406,8 @@ __global__ __launch_bounds__(FLL_THREADS) void k_fft64_long(const double2 *__res
                 default: fl_stage<S, 5, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
             }
         }
-        const int64_t base = (int64_t)line * n;
-        for (int e = tid; e < n; e += FLL_THREADS) {
+        const int64_t base = (int64_t)fl_line(p, line) * n;
+        for (int e = p.r0 + tid; e < p.r0 + p.nr; e += FLL_THREADS) {
             const double2 v = fl_buf[e];
             if constexpr (C64OUT)
                 reinterpret_cast<float2 *>(out)[base + e] = make_float2((float)v.x, (float)v.y);
@@ -475,6 +493,13 @@ int mn_fft64_lines_supported(int64_t n) {
 int mn_fft64_lines(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, const void *in,
                    const double *dec, void *out, int out_c64, int out_layout,
                    mn_stream_t stream) {
+    return mn_fft64_lines_part(A, nin, B, n, isign, in, dec, out, out_c64, out_layout, nullptr,
+                               stream);
+}
+
+int mn_fft64_lines_part(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, const void *in,
+                        const double *dec, void *out, int out_c64, int out_layout,
+                        const int64_t *part, mn_stream_t stream) {
     clear_error();
     MN_REQUIRE(in && out, "fft64_lines: NULL input or output");
     MN_REQUIRE(out_layout >= 0 && out_layout <= 2, "fft64_lines: out_layout must be 0, 1 or 2");
@@ -494,7 +519,29 @@ int mn_fft64_lines(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, cons
         p.ns[s] = ns;
         p.rns[s] = 1.0f / (float)ns;
     }
-    const int nlines = (int)(A * B);
+    // part = {r0, r1, period, q0, q1, c0, c1}; whole rows of lines run on
+    const int64_t all = A * B;
+    int64_t r0 = 0, r1 = n, off = 0, period = all, kc = all, kept = all;
+    if (part) {
+        r0 = part[0], r1 = part[1], period = part[2];
+        const int64_t q0 = part[3], q1 = part[4], c0 = part[5], c1 = part[6];
+        MN_REQUIRE(0 <= r0 && r0 < r1 && r1 <= n, "fft64_lines: bad range of outputs");
+        MN_REQUIRE(period >= 1 && all % period == 0 && (B == 1 || B % period == 0),
+                   "fft64_lines: the period must divide B, or A when B is 1");
+        MN_REQUIRE(0 <= q0 && q0 < q1 && q1 <= all / period && 0 <= c0 && c0 < c1 && c1 <= period,
+                   "fft64_lines: bad range of lines");
+        off = q0 * period + c0;
+        kept = (q1 - q0) * (c1 - c0);
+        kc = c1 - c0;
+        if (kc == period) kc = period = kept;
+    }
+    p.r0 = (int)r0;
+    p.nr = (int)(r1 - r0);
+    p.rnr = 1.0f / (float)p.nr;
+    p.off = (int)off;
+    p.period = (int)period;
+    p.kc = (int)kc;
+    const int nlines = (int)kept;
     // lines up to 4096 long: 512 threads and at most 4096 values (64 KB) per
     // tile, two tiles per CU; longer lines: one line, 1024 threads (the LDS
     // holds one such tile per CU, so its waves are all the latency hiding
@@ -507,8 +554,16 @@ int mn_fft64_lines(int64_t A, int64_t nin, int64_t B, int64_t n, int isign, cons
     // output line stride: B (layout 0), all lines when the line index runs
     // fastest (1), or 1 when each line's values are contiguous (2)
     const int64_t Bo = out_layout == 1 ? A * B : (out_layout == 2 ? 1 : B);
-    int bpow = B > 1 ? __builtin_ctzll((unsigned long long)B) : 30;
-    if (Bo > 1) bpow = min(bpow, (int)__builtin_ctzll((unsigned long long)Bo));
+    // a tile's lines are neighbours within one a: they stay inside a kept row
+    // or, where whole rows are kept, inside aligned runs of B
+    auto pow2 = [](int64_t v) { return v ? (int)__builtin_ctzll((unsigned long long)v) : 30; };
+    int bpow = 30;
+    if (kc != kept) {
+        bpow = pow2(kc);
+    } else {
+        if (B > 1) bpow = min(min(pow2(B), pow2(off)), pow2(kept));
+        if (Bo > 1) bpow = min(min(bpow, pow2(Bo)), pow2(off));
+    }
     while (lti < bpow && (int64_t)(1 << (lti + 1)) <= nlines &&
            n * ((1 << (lti + 1)) + 1) <= vals)
         ++lti;

@@ -26,6 +26,7 @@ targets are set up with their axes in the grid's order. MI355X holds every grid 
 handles in HBM, so there is no slab switch.
 """
 
+import math
 import os
 import warnings
 
@@ -137,6 +138,18 @@ class GpuT3Plan:
         ax = [2, 1, 0] if self.fft_rev else ([1, 2, 0] if self.fft_lines else [0, 1, 2])
         self.grid_shape = [nu[a] for a in ax]
 
+        # cells of each axis that the targets' taps reach: the middle 1 / sigma
+        # and half a kernel width on either side (fp32 coordinates round by an
+        # amount that depends on their offset, and keep the whole axis)
+        self._reach = [(0, n) for n in nu]
+        if self.fft_lines and self._flags & 1:
+            for d in range(3):
+                S = 0.5 * (smax[d] - smin[d])
+                R = S * self.gam[d] * nu[d] / nf[d]
+                far = max(abs(smin[d]), abs(smax[d]))
+                slip = 1e-15 * far / S * R if S > 0.0 else 0.0
+                self._reach[d] = E.target_cells(nu[d], self.w2, R, 1 + int(slip))
+
         # ---- targets: rescale, post factor, bin sort (device fp64) ----------
         stream = E.zstream_eligible(3, self.w2)
         self.bins_trg = (E.make_bins(3, self.w2, self.grid_shape, m=E.ZSTREAM_M) if stream else
@@ -205,8 +218,7 @@ class GpuT3Plan:
         else:
             self.bins_src = E.t3_tile_bins(self.w, self.nf)
         self._hd = hd
-        self._bf = None
-        self._H = None
+        self._bf = self._Hs = self._H64 = self._T = None
         self.low_mem = bool(low_mem) if low_mem is not None else False
         self.set_sources(x64)
 
@@ -254,7 +266,7 @@ class GpuT3Plan:
         if self._bf is None:
             nf, nu = self.nf, self.n_up
             self._bf = torch.empty(nf, dtype=torch.complex128, device=self.device)
-            self._H = torch.empty(self.grid_shape, dtype=torch.complex64, device=self.device)
+            self._Hs = torch.empty(self.grid_shape, dtype=torch.complex64, device=self.device)
             c128 = dict(dtype=torch.complex128, device=self.device)
             if self.fft_rev:
                 self._T = (torch.empty((nu[2], nf[0], nf[1]), **c128),
@@ -268,21 +280,37 @@ class GpuT3Plan:
             else:
                 self._T = None
                 self._H64 = torch.empty(nu, dtype=torch.complex128, device=self.device)
-        return self._bf, self._H, self._H64
+        return self._bf, self._Hs, self._H64
 
-    def _inner_fft(self, bf, H, H64, tm):
-        """H = (complex64) FFT(pad(bf * dec0 x dec1 x dec2)) on the n_up grid."""
+    @property
+    def _H(self):
+        """The whole inner grid of the last execute, from its spread grid: the
+        passes of execute leave out the cells that no target reads. None
+        before the first execute."""
+        if self._bf is None or not self.fft_lines:
+            return self._Hs
+        H = torch.empty_like(self._Hs)
+        self._inner_fft(self._bf, H, None, E.StageTimer(False), reach=[(0, n) for n in self.n_up])
+        return H
+
+    def _inner_fft(self, bf, H, H64, tm, reach=None):
+        """H = (complex64) FFT(pad(bf * dec0 x dec1 x dec2)) on the n_up grid,
+        in the line passes in its cells of reach (the targets' if None) only."""
         nf, nu, d = self.nf, self.n_up, self.dev_dec64
+        kx, ky, kz = reach or self._reach
         if self.fft_rev:
             T1, T2, T3 = self._T
             with tm("fft"):
                 # z lines -> (n2, nf0, nf1); y lines -> (n2, nf0, n1); transpose
                 # -> (n2, n1, nf0); x lines -> H (n2, n1, n0)
+                z0, z1 = kz
                 E.fft64_lines(nf[0] * nf[1], nf[2], 1, nu[2], self.isign, bf, d[2], T1,
-                              layout="lines_last")
-                E.fft64_lines(nu[2] * nf[0], nf[1], 1, nu[1], self.isign, T1, d[1], T2)
-                E.transpose_c128(nu[2], nf[0], nu[1], T2, T3)
-                E.fft64_lines(nu[2] * nu[1], nf[0], 1, nu[0], self.isign, T3, d[0], H)
+                              layout="lines_last", keep=kz)
+                E.fft64_lines(nu[2] * nf[0], nf[1], 1, nu[1], self.isign, T1, d[1], T2, keep=ky,
+                              rows=(nf[0], kz, (0, nf[0])))
+                E.transpose_c128(z1 - z0, nf[0], nu[1], T2[z0:z1], T3[z0:z1])
+                E.fft64_lines(nu[2] * nu[1], nf[0], 1, nu[0], self.isign, T3, d[0], H, keep=kx,
+                              rows=(nu[1], kz, ky))
             return
         if self.fft_lines:
             T1, T2 = self._T
@@ -291,10 +319,11 @@ class GpuT3Plan:
                 # -> H (n1, n2, n0), each x line stored whole: 2.31 against
                 # 2.55 ms for the x pass at 640^3 when the strided x lines
                 # were stored in place (runs of 4 complex64 values)
-                E.fft64_lines(nf[0] * nf[1], nf[2], 1, nu[2], self.isign, bf, d[2], T1)
-                E.fft64_lines(nf[0], nf[1], nu[2], nu[1], self.isign, T1, d[1], T2)
+                E.fft64_lines(nf[0] * nf[1], nf[2], 1, nu[2], self.isign, bf, d[2], T1, keep=kz)
+                E.fft64_lines(nf[0], nf[1], nu[2], nu[1], self.isign, T1, d[1], T2, keep=ky,
+                              rows=(nu[2], (0, nf[0]), kz))
                 E.fft64_lines(1, nf[0], nu[1] * nu[2], nu[0], self.isign, T2, d[0], H,
-                              layout="lines_first")
+                              layout="lines_first", keep=kx, rows=(nu[2], ky, kz))
             return
         with tm("pad+deconv"):
             E.pad_deconv_c128(self.n_up, self.nf, bf, d, H64)
@@ -324,7 +353,7 @@ class GpuT3Plan:
             else:
                 E.interp(self.trg, self.beta2, H, out, post=self.trg.extra)
         if self.low_mem:
-            self._bf = self._H = self._H64 = self._T = None
+            self._bf = self._Hs = self._H64 = self._T = None
         return out
 
     def _strengths(self, c):

@@ -17,7 +17,7 @@
 //
 // One workgroup holds TI whole lines in LDS (n <= 8192, so a line of 7200
 // doubles fits where the runtime's transform splits it into several passes)
-// and runs mixed-radix Stockham stages of radix 8, 4, 2, 3 and 5 over them;
+// and runs mixed-radix Stockham stages of radix 2 to 12 over them;
 // each stage reads its butterflies into registers, waits at a barrier and
 // writes them back in place. The twiddle exp(isign 2 pi i m / n) for each
 // butterfly comes from a per-(device, n, sign) table computed once with fp64
@@ -50,6 +50,7 @@ namespace {
 
 constexpr int FL_NMAX = 8192;   // longest line: 128 KB of LDS
 constexpr int FL_WIDE = 5120;   // values of an unpadded strided tile (80 KB)
+constexpr int FL_SHORT = 4096;  // longest line of the tiles of 512 threads
 constexpr int FL_MAXST = 16;
 
 // ti = 2^lti lines per tile, stored element-major in LDS (value p of line l
@@ -170,12 +171,39 @@ __device__ __forceinline__ void ddft5(double2 *v) {
 }
 
 template <int S, int R>
+__device__ __forceinline__ void ddft(double2 *v);
+
+// R = A B with coprime A and B: over the inputs (a B + b A) mod R the DFT
+// splits into A- and B-point DFTs without twiddles, output k at (k mod A,
+// k mod B) (Good, 1958).
+template <int S, int A, int B>
+__device__ __forceinline__ void ddft_coprime(double2 *v) {
+    double2 y[A][B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        double2 t[A];
+#pragma unroll
+        for (int a = 0; a < A; ++a) t[a] = v[(a * B + b * A) % (A * B)];
+        ddft<S, A>(t);
+#pragma unroll
+        for (int a = 0; a < A; ++a) y[a][b] = t[a];
+    }
+#pragma unroll
+    for (int a = 0; a < A; ++a) ddft<S, B>(y[a]);
+#pragma unroll
+    for (int k = 0; k < A * B; ++k) v[k] = y[k % A][k % B];
+}
+
+template <int S, int R>
 __device__ __forceinline__ void ddft(double2 *v) {
     if constexpr (R == 2) ddft2<S>(v);
     else if constexpr (R == 3) ddft3<S>(v);
     else if constexpr (R == 4) ddft4<S>(v);
     else if constexpr (R == 5) ddft5<S>(v);
-    else ddft8<S>(v);
+    else if constexpr (R == 6) ddft_coprime<S, 2, 3>(v);
+    else if constexpr (R == 8) ddft8<S>(v);
+    else if constexpr (R == 10) ddft_coprime<S, 2, 5>(v);
+    else ddft_coprime<S, 4, 3>(v);
 }
 
 // One Stockham stage of radix R over the ti lines of n values in LDS,
@@ -201,13 +229,16 @@ __device__ __forceinline__ void fl_stage(double2 *buf, const double2 *__restrict
             const int l = b & lmask, j = b >> lti;
             const int k = j - fdiv(j, Ns, rNs) * Ns;
             const double2 *src = buf + j * ts + l;
-            v[f][0] = src[0];
-            const double2 w = tw[k * tws];
-            double2 wr = w;
 #pragma unroll
-            for (int r = 1; r < R; ++r) {
-                v[f][r] = dmul(src[r * nr * ts], wr);
-                if (r + 1 < R) wr = dmul(wr, w);
+            for (int r = 0; r < R; ++r) v[f][r] = src[r * nr * ts];
+            const double2 w = tw[k * tws];
+            if (Ns > 1) {  // the first stage has no twiddles
+                double2 wr = w;
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    v[f][r] = dmul(v[f][r], wr);
+                    if (r + 1 < R) wr = dmul(wr, w);
+                }
             }
             ddft<S, R>(v[f]);
         }
@@ -227,12 +258,43 @@ __device__ __forceinline__ void fl_stage(double2 *buf, const double2 *__restrict
     __syncthreads();
 }
 
+// All stages of the plan: bound by the latency of a stage (two tiles share a
+// CU), so composite radices take one stage out: lines of 640 points run 10, 8, 8
+// instead of 5, 8, 8, 2, and the 640^3 passes z + y 2131 -> 1949 us, x
+// 1225 -> 1114; 240 points 10, 6, 4 instead of 5, 3, 8, 2, 210 -> 193 us. Radix
+// 12 and 128 registers keep both tiles resident (15 and 16 need 151). Tiles of
+// one long line (T = 1024) keep radices 8 and below: 12, 10 and 6 spill there.
+template <int S, int T, int VALS>
+__device__ __forceinline__ void fl_stages(double2 *buf, const double2 *__restrict__ tw,
+                                          const FlPlan &p, int lti, int ts, int tid) {
+    const int n = p.n;
+    for (int s = 0; s < p.nst; ++s) {
+        const int Ns = p.ns[s];
+        const float rNs = p.rns[s];
+        if constexpr (T <= 512) {
+            switch (p.rad[s]) {
+                case 12: fl_stage<S, 12, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); continue;
+                case 10: fl_stage<S, 10, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); continue;
+                case 6: fl_stage<S, 6, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); continue;
+                default: break;
+            }
+        }
+        switch (p.rad[s]) {
+            case 8: fl_stage<S, 8, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); break;
+            case 5: fl_stage<S, 5, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); break;
+            case 4: fl_stage<S, 4, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); break;
+            case 3: fl_stage<S, 3, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); break;
+            default: fl_stage<S, 2, T, VALS>(buf, tw, n, lti, ts, Ns, rNs, tid); break;
+        }
+    }
+}
+
 // T threads, at most VALS values (ti * n) per tile. With B == 1 the tile's
 // lines are consecutive runs of the input and output; with B > 1, ti divides
 // B or the kept part of it, so the tile's lines share a and element m of all
 // of them is ti contiguous values.
 template <int S, bool C64OUT, int T, int VALS>
-__global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ in,
+__global__ __launch_bounds__(T, 4) void k_fft64_lines(const double2 *__restrict__ in,
                                                    void *__restrict__ out,
                                                    const double *__restrict__ dec,
                                                    const double2 *__restrict__ tw, int nlines,
@@ -295,17 +357,7 @@ __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ i
         }
     }
     __syncthreads();
-    for (int s = 0; s < p.nst; ++s) {
-        const int Ns = p.ns[s];
-        const float rNs = p.rns[s];
-        switch (p.rad[s]) {
-            case 8: fl_stage<S, 8, T, VALS>(fl_buf, tw, n, lti, ts, Ns, rNs, tid); break;
-            case 4: fl_stage<S, 4, T, VALS>(fl_buf, tw, n, lti, ts, Ns, rNs, tid); break;
-            case 2: fl_stage<S, 2, T, VALS>(fl_buf, tw, n, lti, ts, Ns, rNs, tid); break;
-            case 3: fl_stage<S, 3, T, VALS>(fl_buf, tw, n, lti, ts, Ns, rNs, tid); break;
-            default: fl_stage<S, 5, T, VALS>(fl_buf, tw, n, lti, ts, Ns, rNs, tid); break;
-        }
-    }
+    fl_stages<S, T, VALS>(fl_buf, tw, p, lti, ts, tid);
     auto put = [&](int64_t o, double2 v) {
         if constexpr (C64OUT)
             reinterpret_cast<float2 *>(out)[o] = make_float2((float)v.x, (float)v.y);
@@ -318,7 +370,7 @@ __global__ __launch_bounds__(T) void k_fft64_lines(const double2 *__restrict__ i
         const int cnt = min(ti, nlines - k0) * nr;
         for (int e = tid; e < cnt; e += T) {
             const int l = fdiv(e, nr, p.rnr), r = e - l * nr;
-            put(base + (int64_t)l * n + r, fl_buf[(r0 + r) * ts + l]);
+            put(base + (l * n + r), fl_buf[(r0 + r) * ts + l]);
         }
     } else {
         const int a = li0 / Bo, b0 = li0 - a * Bo;
@@ -395,17 +447,7 @@ __global__ __launch_bounds__(FLL_THREADS) void k_fft64_long(const double2 *__res
         __syncthreads();
         const int nl = line + gridDim.x;
         if (nl < nlines) load(nl);
-        for (int st = 0; st < p.nst; ++st) {
-            const int Ns = p.ns[st];
-            const float rNs = p.rns[st];
-            switch (p.rad[st]) {
-                case 8: fl_stage<S, 8, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
-                case 4: fl_stage<S, 4, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
-                case 2: fl_stage<S, 2, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
-                case 3: fl_stage<S, 3, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
-                default: fl_stage<S, 5, FLL_THREADS, FL_NMAX>(fl_buf, tw, n, 0, 1, Ns, rNs, tid); break;
-            }
-        }
+        fl_stages<S, FLL_THREADS, FL_NMAX>(fl_buf, tw, p, 0, 1, tid);
         const int64_t base = (int64_t)fl_line(p, line) * n;
         for (int e = p.r0 + tid; e < p.r0 + p.nr; e += FLL_THREADS) {
             const double2 v = fl_buf[e];
@@ -427,26 +469,27 @@ __global__ void k_fl_twiddles(double2 *tw, int n, int S) {
     tw[m] = make_double2(c, S * s);
 }
 
-// Radices for n = 2^a 3^b 5^c, largest stages first; 0 if n has another
-// factor or needs more than FL_MAXST stages.
-int fl_radices(int64_t n, int *rad) {
-    int ns = 0;
-    int64_t m = n;
-    for (int R : {5, 3}) {
-        while (m % R == 0) {
-            if (ns == FL_MAXST) return 0;
-            rad[ns++] = R;
-            m /= R;
+// Radices for n = 2^a 3^b 5^c: as few stages as the radices allow, then the
+// smallest ones. Odd ones go first: the first stage's stores are its radix
+// apart, and even strides share LDS banks. 0 if n has another factor or needs more than FL_MAXST stages.
+int fl_radices(int64_t n, int *rad, int most = FL_MAXST, int top = 12, bool six = true) {
+    if (n == 1) return 0;
+    int best = 0, sum = 0, cur[FL_MAXST];
+    for (int R : {12, 10, 8, 6, 5, 4, 3, 2}) {
+        if (R > top || (R == 6 && !six) || n % R || most < 1) continue;
+        cur[0] = R;
+        const int rest = n == R ? 0 : fl_radices(n / R, cur + 1, most - 1, R, six);
+        if (n != R && !rest) continue;
+        int cs = 0;
+        for (int i = 0; i <= rest; ++i) cs += cur[i];
+        if (!best || rest + 1 < best || (rest + 1 == best && cs < sum)) {
+            best = rest + 1;
+            sum = cs;
+            std::copy(cur, cur + best, rad);
+            most = best;  // no more stages than this from here on
         }
     }
-    for (int R : {8, 4, 2}) {
-        while (m % R == 0) {
-            if (ns == FL_MAXST) return 0;
-            rad[ns++] = R;
-            m /= R;
-        }
-    }
-    return m == 1 ? ns : 0;
+    return best;
 }
 
 std::mutex g_tw_mu;
@@ -512,7 +555,8 @@ int mn_fft64_lines_part(int64_t A, int64_t nin, int64_t B, int64_t n, int isign,
     FlPlan p{};
     p.n = (int)n;
     p.nin = (int)nin;
-    p.nst = fl_radices(n, p.rad);
+    p.nst = fl_radices(n, p.rad, FL_MAXST, n > FL_SHORT ? 8 : 12, n <= FL_SHORT);
+    std::stable_partition(p.rad, p.rad + p.nst, [](int r) { return r % 2; });
     p.rn = 1.0f / (float)n;
     p.rnin = 1.0f / (float)nin;
     for (int s = 0, ns = 1; s < p.nst; ns *= p.rad[s], ++s) {
@@ -548,7 +592,7 @@ int mn_fft64_lines_part(int64_t A, int64_t nin, int64_t B, int64_t n, int isign,
     // there is). Measured on MI355X: 640^3 passes 5.70 ms with 512 threads,
     // 6.59 with 256, 7.8 with 1024; 7200-point lines of a 7200^2 x 24 grid
     // 11.3 ms with 1024 threads, 13.8 with 512.
-    const bool longl = n > 4096;
+    const bool longl = n > FL_SHORT;
     const int vals = longl ? 8192 : 4096;
     int lti = 0;
     // output line stride: B (layout 0), all lines when the line index runs

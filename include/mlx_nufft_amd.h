@@ -303,7 +303,8 @@ int mn_interp_zgather(const mn_bins *g, float beta, int64_t P, int64_t B, int zs
  * to be added to cell x - n[d], as mn_fftg_crop_deconv does), and
  * mn_interp_zgather_ext reads such grids with their images filled in
  * (mn_fftg_pad_deconv). Both evaluate the kernel's exponent without
- * cancellation. mn_zsweep_maxload writes the largest number of points one
+ * cancellation, and mn_interp_zgather_ext also serves the words and grids of
+ * mn_interp_zgather that way. mn_zsweep_maxload writes the largest number of points one
  * wavefront of a sweep in segments of zseg visits (device int32), which bounds
  * the sweep's time where points crowd.
  * ref: nd.py:152-165, nd.py:492-579, nd.py:974-1073.

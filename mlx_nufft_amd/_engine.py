@@ -338,9 +338,10 @@ class ZSweepPoints:
     same P and geometry, its device buffers are reused, so re-pointing
     allocates nothing; prev's contents are overwritten in stream order.
     ngrid: the periodic grid when bins describe larger extents (then ext is
-    True and every footprint lies inside them)."""
+    True and every footprint lies inside them). stable: the gather evaluates
+    its weights without cancellation (always on extents)."""
 
-    def __init__(self, bins, x64, prec64, prev=None, gather=False, ngrid=None):
+    def __init__(self, bins, x64, prec64, prev=None, gather=False, ngrid=None, stable=False):
         lib = L.lib()
         dev = x64[0].device
         self.kind = "zgather" if gather else "zsweep"
@@ -359,6 +360,7 @@ class ZSweepPoints:
         word = buf("word_in", P, torch.int32)
         fr = buf("fr_in", (3, P), torch.float32)
         self.ext = ngrid is not None
+        self.stable = stable
         self.zseg = zsweep_segment([int(bins.n[d]) for d in range(3)])
         L.check(lib.mn_zsweep_setpts_ext(ctypes.byref(bins), L.i64x3(ngrid), int(gather), P,
                                          L.ptr3(x64), int(bool(prec64)), L.ptr(word),
@@ -735,7 +737,7 @@ def interp_direct_preferred(pts, w, n_up):
     return direct < 5.0 * staged
 
 
-def zgather_preferred(P, w, n_up):
+def zgather_preferred(P, w, n_up, sigma=2.0):
     """True when the z-gather interpolation should beat the direct and the
     staged-tile gathers for P points on the 3D fine grid n_up. The direct
     gather reads P w^3 taps, the z-gather (8 + w - 1)^2 columns of 8 new
@@ -748,23 +750,44 @@ def zgather_preferred(P, w, n_up):
     taps. Measured, us, z-gather / tiles: 384 x 400 x 432, 2e6 points, w = 4
     341 / 266, w = 5 349 / 420, w = 8 439 / 866; 200 x 192 x 180, 1.4e6, w = 4
     93 / 67, w = 5 98 / 75, w = 6 104 / 104, w = 8 141 / 235; 1.1e7, w = 5
-    555 / 672. (Below 2^18 points the w <= 5 difference is some us.)"""
+    555 / 672. (Below 2^18 points the w <= 5 difference is some us.)
+    Between the factors the other gathers read the grid in fp32, so there the
+    z-gather's split operands need the weights that make up for them
+    (zgather_stable), and below sigma = 2 they do not: 2e6 points on 360^3 at
+    sigma = 1.25, w = 7, 1.5048e-4 from 64 bits against 1.5044e-4."""
+    ratio = _zgather_ratio(P, w, n_up)
+    cells = float(n_up[0]) * float(n_up[1]) * float(n_up[2])
+    if cells >= 2.0 ** 25:
+        return ratio >= (1.5 if sigma >= 2.0 else 5.0)
+    if w <= 5 and P >= 1 << 18 and (w < 5 or P < 1.2 * cells):
+        return False
+    return ratio >= 5.0
+
+
+def _zgather_ratio(P, w, n_up):
+    """Taps of the direct gather over the cells the z-gather reads."""
     nchunks = (n_up[0] / 8.0) * (n_up[1] / 8.0) * -(-n_up[2] // 8)
     lam = float(P) / nchunks
     busy = nchunks * -np.expm1(-lam)
-    staged = (8 + w - 1) ** 2 * 8.0 * busy * (1.0 + np.exp(-lam))
-    cells = float(n_up[0]) * float(n_up[1]) * float(n_up[2])
-    if cells >= 2.0 ** 25:
-        return float(P) * w ** 3 >= 1.5 * staged
-    if w <= 5 and P >= 1 << 18 and (w < 5 or P < 1.2 * cells):
-        return False
-    return float(P) * w ** 3 >= 5.0 * staged
+    return float(P) * w ** 3 / ((8 + w - 1) ** 2 * 8.0 * busy * (1.0 + np.exp(-lam)))
+
+
+def zgather_stable(P, w, n_up):
+    """Whether a z-gather on its own grid evaluates the kernel's exponent
+    without cancellation: where it takes points from the fp32 gathers (below
+    the factor 5 of zgather_preferred) it must be no further from 64 bits
+    than they are. 3e6 points on 384^3, z-gather / with this exponent / fp32
+    gather: w = 6 1.1950e-5 / 1.1933e-5 / 1.1944e-5, w = 7 1.620e-6 / 1.438e-6
+    / 1.578e-6, w = 8 8.64e-7 / 3.43e-7 / 7.89e-7; the times are equal
+    (787 and 780 us at w = 7)."""
+    return _zgather_ratio(P, w, n_up) < 5.0
 
 
 def interp_zgather(pts, beta, grids, outs, B=1, zseg=None):
     """3D interpolation over the z-sweep point state: B grids (B x n_up)
     into B output vectors of P values in caller order (outs: B x P)."""
-    fn = L.lib().mn_interp_zgather_ext if pts.ext else L.lib().mn_interp_zgather
+    stable = pts.ext or pts.stable
+    fn = L.lib().mn_interp_zgather_ext if stable else L.lib().mn_interp_zgather
     L.check(fn(ctypes.byref(pts.bins), float(beta), pts.P, int(B), int(zseg or pts.zseg),
                L.ptr(pts.zstart), L.ptr(pts.perm), L.ptr(pts.word), L.ptr3(pts.fr_rows()),
                L.ptr(grids), L.ptr(outs), L.stream()), "interp_zgather")

@@ -230,7 +230,9 @@ class _PointsND:
                 same = isinstance(prev, E.ZSweepPoints) and prev.kind == kind
                 self.pts = E.ZSweepPoints(self._zbins, x64, prec64, prev=prev if same else None,
                                           gather=self._zgather_points,
-                                          ngrid=self.n_up if self._ext else None)
+                                          ngrid=self.n_up if self._ext else None,
+                                          stable=self._zgather_points and
+                                          E.zgather_stable(self.P, self.w, self.n_up))
             del prev
             many = self._ymfma if self._ysweep else True
             many = many and self.P >= 1 << (17 if self._ysweep else 18)
@@ -530,7 +532,7 @@ class Type2PlanND(_PointsND):
             return False
         if os.environ.get("MN_INTERP", "") in ("tiles", "zstream"):
             return False
-        return E.zgather_preferred(self.P, self.w, self.n_up)
+        return E.zgather_preferred(self.P, self.w, self.n_up, self.sigma)
 
     def _gather_direct(self):
         """3D points sparse on the fine grid read their taps directly (no

@@ -321,11 +321,25 @@ _SWEEP_RATES = {"zsweep": (20.0, 0.04), "zgather": (8.0, 0.017), "ymfma": (21.0,
 
 def sweep_balanced(load, kind, w, P, slack=1.0):
     """Whether a sweep is not held up by crowded points: its time is at least
-    that of its most loaded wave, which should not exceed slack times what the
-    tile kernels take for all points. Reads load back (4 bytes, as the tile
-    path's subproblem count)."""
+    that of its most loaded wave (load points), which should not exceed slack
+    times what the tile kernels take for all points."""
     per_us, tile_us = _SWEEP_RATES[kind]
-    return load.item() / per_us <= slack * (30.0 + tile_us * 1e-3 * w * P)
+    return load / per_us <= slack * (30.0 + tile_us * 1e-3 * w * P)
+
+
+def sweep_sums_short(load, w, zseg):
+    """Whether fp32 sums of the most loaded wave (load points) stay as near to
+    64 bits as the tiles' fp64 sums of fp32 weights were. They add 1.6e-7 times
+    the root of the points per cell: none of the error up to w = 5, as much as
+    the tiles had at 20 points a cell for w = 6 (1.164e-5 both) and past 8 for
+    wider kernels. Relative errors at 0.3 / 3 / 8 / 20 points per cell, 90 x 100
+    x 120, against those tiles: w = 8 2.9e-7 / 3.9e-7 / 5.3e-7 / 7.7e-7 and
+    6.9e-7 to 7.0e-7, w = 7 1.32e-6 / 1.35e-6 / 1.38e-6 / 1.45e-6 and 1.45e-6.
+    The bound is the load of so many points spread evenly."""
+    if w <= 5:
+        return True
+    per_cell = 20.0 if w == 6 else 8.0
+    return load <= per_cell * 64.0 * (zseg + 8) * ((8 + w - 1) / 8.0) ** 2
 
 
 class ZSweepPoints:

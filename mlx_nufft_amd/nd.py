@@ -249,7 +249,11 @@ class _PointsND:
         2625 / 135; 2D, w = 7, 1e6 on 1024^2 455 / 90, 5e6 on 2048^2
         1507 / 282."""
         slack = 1.0 if self._ext else (2.0 if self._ysweep else 3.0)
+        load = load.item()  # 4 bytes, as the tile path's subproblem count
         self._crowded = not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack)
+        if self._ext and self.pts.kind == "zsweep" and not self._crowded:
+            # grids whose other route sums in fp64
+            self._crowded = not E.sweep_sums_short(load, self.w, self.pts.zseg)
         return not self._crowded
 
     def _store(self):

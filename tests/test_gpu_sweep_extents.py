@@ -135,3 +135,66 @@ def test_crowded_points_2d(mn):
         assert np.linalg.norm(p.execute(c) - ref) <= 3e-6 * np.linalg.norm(ref)
     q = mn.Type1PlanND(wide, (128, 135), eps=eps)     # 256 x 270
     assert q.pts.kind == "tiles"
+
+
+def _sums64(x, c, f, N, ntrg):
+    """Direct type-1 sums, and type-2 sums at the first ntrg points, in 64 bits."""
+    step = 8192
+    t1 = torch.zeros(N[0] * N[1], N[2], dtype=torch.complex128, device="cuda")
+    t2 = []
+    fd = torch.from_numpy(f).cuda().to(torch.complex128).reshape(N[0], -1)
+    for lo in range(0, x[0].size, step):
+        e = []
+        for d in range(3):
+            k = torch.arange(-(N[d] // 2), N[d] - N[d] // 2, dtype=torch.float64, device="cuda")
+            ph = torch.from_numpy(x[d][lo:lo + step]).cuda()[:, None] * k
+            e.append(torch.complex(torch.cos(ph), torch.sin(ph)))
+        cd = torch.from_numpy(c[lo:lo + step]).cuda().to(torch.complex128)
+        xy = (e[0][:, :, None] * (cd[:, None] * e[1])[:, None, :]).reshape(cd.numel(), -1)
+        t1 += xy.T.contiguous() @ e[2]
+        if lo < ntrg:
+            g = (e[0].conj().contiguous() @ fd).reshape(-1, N[1], N[2])
+            t2.append(((g * e[1].conj()[:, :, None]).sum(1) * e[2].conj()).sum(1))
+    return t1.reshape(N), torch.cat(t2)[:ntrg]
+
+
+# eps, points per cell, most allowed relative error: what fp64 tile sums of
+# fp32 weights gave here (1.45e-6 at w = 7, 6.9e-7 to 7.3e-7 at w = 8)
+@pytest.mark.parametrize("eps,dens,most", [(1e-6, 0.3, 1.46e-6), (1e-6, 6.0, 1.46e-6),
+                                           (1e-7, 0.3, 7.3e-7), (1e-7, 6.0, 7.3e-7)])
+def test_extents_no_less_precise_than_fp64_sums(eps, dens, most, mn):
+    """Split products and fp32 sums on extents against 64 bits, with strengths
+    and modes of one size and over a range of e^+-12: no further off than fp64
+    sums of fp32 weights on the periodic grid."""
+    print(f"case extents precision eps={eps} points per cell {dens}", flush=True)
+    rng = np.random.default_rng(36)
+    N = (45, 50, 55)                                      # 90 x 100 x 120
+    M, T = int(dens * 90 * 100 * 120), 65536
+    x = _pts(rng, M)
+    for wide in (False, True):
+        c, f = _cplx(rng, M), _cplx(rng, N)
+        if wide:
+            c *= np.exp(4 * rng.standard_normal(M)).astype(np.float32)
+            f *= np.exp(4 * rng.standard_normal(N)).astype(np.float32)
+        e1, e2 = _sums64(x, c, f, N, T)
+        p, g = mn.Type1PlanND(x, N, eps=eps), mn.Type2PlanND(x, N, eps=eps)
+        assert p.n_up == [90, 100, 120] and p._store() is not None and g._store() is not None
+        r = [float((a.to(torch.complex128) - b).norm() / b.norm()) for a, b in
+             ((p.execute(c, return_np=False), e1), (g.execute(f, return_np=False)[:T], e2))]
+        print(f"  wide={wide} type 1 {r[0]:.3e} type 2 {r[1]:.3e}", flush=True)
+        assert max(r) <= most
+
+
+def test_extents_leave_dense_sets_to_fp64_sums(mn):
+    """fp32 sums lose to the tiles' fp64 ones where a cell sums many points
+    (7.7e-7 against 7.0e-7 at 20 a cell, w = 8), so from 8 a cell on the tiles
+    have them, on re-pointing as on a new plan."""
+    print("case extents dense", flush=True)
+    rng = np.random.default_rng(37)
+    N, cells = (45, 50, 55), 90 * 100 * 120
+    thin, dense = _pts(rng, 6 * cells), _pts(rng, 12 * cells)
+    p = mn.Type1PlanND(dense, N, eps=1e-7)
+    assert p.pts.kind == "tiles" and p._store() is None
+    for x, kind in ((thin, "zsweep"), (dense, "tiles")):
+        p.set_sources(x)
+        assert p.pts.kind == kind

@@ -126,7 +126,7 @@ class _PointsND:
             self._ysweep = False
         if self._ysweep:
             self._ybins = E.make_bins(2, self.w, self.n_up, m=(16 if self._ymfma else 64, 1))
-        load = self._set_points(x64, defer=True)
+        load = self._set_points(x64, building=True)
 
         # Mode deconvolution 1/phihat(2 pi k / n_up) on the uncentred fine grid
         # (points folded into [0, 2pi), so no (-1)^k factor). rocFFT's backward
@@ -139,6 +139,7 @@ class _PointsND:
         self._work = None
         # the rest of the plan was queued behind the sort; now look at its result
         if load is not None and not self._uncrowded(load):
+            self._watch = not self._ext
             self.pts = None
             self._set_points(x64, tiles=True)
 
@@ -184,15 +185,15 @@ class _PointsND:
         self.i1 = [v.cpu().numpy() for v in i1]
         self.fr = [v.cpu().numpy() for v in fr]
 
-    def _set_points(self, x64, defer=False, tiles=False):
+    def _set_points(self, x64, building=False, tiles=False):
         """Build the point state. Where a sweep has to be looked at for
-        crowding and defer is set, its load is returned for the caller to look
-        at once it has time; tiles builds the tiles' state."""
+        crowding while the plan is built, its load is returned for the caller
+        to look at once it has time; tiles builds the tiles' state."""
         tm = self._timer()
         load = None
         if (self._zsweep or self._ext or self._ysweep) and not tiles:
-            load = self._set_sweep_points(x64, tm)
-            if load is not None and not defer and not self._uncrowded(load):
+            load = self._set_sweep_points(x64, tm, building)
+            if load is not None and not building and not self._uncrowded(load):
                 self.pts = None
                 return self._set_points(x64, tiles=True)
         else:
@@ -208,16 +209,16 @@ class _PointsND:
         self.last_setpts_profile = dict(self.last_profile) if self.profile else {}
         return load
 
-    # whether the points of the last set held the sweep up (None: no set yet)
-    _crowded = None
+    # whether a plan on a sweep's own grid was built on points that crowd
+    _watch = False
 
-    def _set_sweep_points(self, x64, tm):
+    def _set_sweep_points(self, x64, tm, building):
         """Point state of a sweep or the z-gather. Returns its load where the
-        points may hold it up, else None: every set on grids stored with
-        extents; on the sweeps' own grids, where re-pointing reads nothing
-        back and results do not depend on the order of atomics, the first set
-        of 2^18 points (2^17 in 2D) or more, and further ones while they are
-        crowded."""
+        set has to be looked at for crowding, else None. On grids stored with
+        extents every set is; on the sweeps' own grids the plan's first set is,
+        from 2^18 points on (2^17 in 2D), and further ones if that one crowded:
+        other plans' re-pointing reads nothing back, so that a program whose
+        points move need not wait for the device, and stays with the sweep."""
         prec64 = self.prec == "crit64"
         with tm("setpts+sort+tables"):
             prev = getattr(self, "pts", None)
@@ -236,10 +237,8 @@ class _PointsND:
             del prev
             many = self._ymfma if self._ysweep else True
             many = many and self.P >= 1 << (17 if self._ysweep else 18)
-            if self._ext or (self._crowded is not False and many):
+            if self._ext or ((building or self._watch) and many):
                 return E.sweep_load(self.pts)
-        if self._crowded is None:
-            self._crowded = False
         return None
 
     def _uncrowded(self, load):
@@ -250,11 +249,11 @@ class _PointsND:
         1507 / 282."""
         slack = 1.0 if self._ext else (2.0 if self._ysweep else 3.0)
         load = load.item()  # 4 bytes, as the tile path's subproblem count
-        self._crowded = not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack)
-        if self._ext and self.pts.kind == "zsweep" and not self._crowded:
-            # grids whose other route sums in fp64
-            self._crowded = not E.sweep_sums_short(load, self.w, self.pts.zseg)
-        return not self._crowded
+        if not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack):
+            return False
+        # on extents the other route's sums are fp64 ones
+        return (not self._ext or self.pts.kind != "zsweep"
+                or E.sweep_sums_short(load, self.w, self.pts.zseg))
 
     def _store(self):
         """Extents the fine grid is stored with (None: n_up) for these points."""

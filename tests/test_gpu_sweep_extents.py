@@ -198,3 +198,47 @@ def test_extents_leave_dense_sets_to_fp64_sums(mn):
     for x, kind in ((thin, "zsweep"), (dense, "tiles")):
         p.set_sources(x)
         assert p.pts.kind == kind
+
+
+@pytest.mark.parametrize("N,M,sweep", [((32, 32, 32), 1 << 18, "zsweep"),
+                                       ((128, 128), 1 << 17, "ymfma")])
+def test_native_route_depends_on_first_and_current_set_only(N, M, sweep, mn):
+    """On the sweeps' own grids a plan built on crowded points looks at every
+    set, also after ones that were spread out; a plan built on others, few
+    points among them, reads nothing back and stays with the sweep. Results
+    are those of the tiles."""
+    print(f"case native route N={N}", flush=True)
+    rng = np.random.default_rng(38)
+    dim = len(N)
+    dev = lambda x: tuple(torch.from_numpy(v).cuda() for v in x)
+    crowd = dev([rng.uniform(0.1, 0.2, M) for _ in range(dim)])
+    wide = dev([rng.uniform(-np.pi, np.pi, M) for _ in range(dim)])
+    few = tuple(v[:1000].contiguous() for v in wide)
+    c = _cplx(rng, M)
+    ref = {k: mn.Type1PlanND(x, N, eps=1e-6, spread_method="gm").execute(c)
+           for k, x in (("crowd", crowd), ("wide", wide))}
+
+    # a sweep adds a cell's points one after another in fp32: each of the M
+    # additions to the crowd's few cells rounds by up to 2^-24 of a partial sum
+    # that grows as its root, sqrt(M / 2) 2^-24 of the whole in all
+    swept = 2.0 ** -24 * np.sqrt(M / 2)
+
+    def check(p, key):
+        a = p.execute(c)
+        tol = 3e-6 if key == "wide" or p.pts.kind == "tiles" else swept
+        assert np.linalg.norm(a - ref[key]) <= tol * np.linalg.norm(ref[key])
+
+    p = mn.Type1PlanND(crowd, N, eps=1e-6)
+    for key, x, kind in (("wide", wide, sweep), ("crowd", crowd, "tiles"), ("wide", wide, sweep)):
+        p.set_sources(x)
+        assert p.pts.kind == kind
+        check(p, key)
+    for first in (wide, few):
+        p = mn.Type1PlanND(first, N, eps=1e-6)
+        torch.cuda.set_sync_debug_mode("error")
+        try:
+            p.set_sources(crowd)
+        finally:
+            torch.cuda.set_sync_debug_mode("default")
+        assert p.pts.kind == sweep
+        check(p, "crowd")

@@ -319,12 +319,17 @@ def sweep_load(pts):
 _SWEEP_RATES = {"zsweep": (20.0, 0.04), "zgather": (8.0, 0.017), "ymfma": (21.0, 0.012)}
 
 
-def sweep_balanced(load, kind, w, P, slack=1.0):
+def sweep_balanced(load, kind, w, P, slack=1.0, repoint=False):
     """Whether a sweep is not held up by crowded points: its time is at least
     that of its most loaded wave (load points), which should not exceed slack
-    times what the tile kernels take for all points."""
+    times what the tile kernels take for all points. A step that re-points a
+    plan also pays for the tiles' own point state after the sweep's (us, set
+    and transform with the tiles / the sweep, radial points: 2D, w = 7, 1e6 on
+    2048^2 472 / 387, 3e5 398 / 218; 3D, w = 2, 3e4 on 90 x 100 x 120
+    310 / 203): 165 us and 30 for every 1e6 points more."""
     per_us, tile_us = _SWEEP_RATES[kind]
-    return load / per_us <= slack * (30.0 + tile_us * 1e-3 * w * P)
+    setup = 165.0 + 30e-6 * P if repoint else 0.0
+    return load / per_us <= slack * (30.0 + tile_us * 1e-3 * w * P) + setup
 
 
 def sweep_sums_short(load, w, zseg):

@@ -139,7 +139,15 @@ class _PointsND:
         self._work = None
         # the rest of the plan was queued behind the sort; now look at its result
         if load is not None and not self._uncrowded(load):
-            self._watch = not self._ext
+            # On extents such a plan is one of tiles from now on: building the
+            # sweep's state for every set first would cost small transforms more
+            # than the sweep saves (a step of 1e5 crowded points on 54 x 50 x 72,
+            # w = 4: 209 us without it, 294 with). On the sweep's own grids, where
+            # spread-out sets are worth far more, it goes on looking.
+            if self._ext:
+                self._ext = None
+            else:
+                self._watch = True
             self.pts = None
             self._set_points(x64, tiles=True)
 
@@ -193,7 +201,7 @@ class _PointsND:
         load = None
         if (self._zsweep or self._ext or self._ysweep) and not tiles:
             load = self._set_sweep_points(x64, tm, building)
-            if load is not None and not building and not self._uncrowded(load):
+            if load is not None and not building and not self._uncrowded(load, repoint=True):
                 self.pts = None
                 return self._set_points(x64, tiles=True)
         else:
@@ -215,7 +223,8 @@ class _PointsND:
     def _set_sweep_points(self, x64, tm, building):
         """Point state of a sweep or the z-gather. Returns its load where the
         set has to be looked at for crowding, else None. On grids stored with
-        extents every set is; on the sweeps' own grids the plan's first set is,
+        extents every set is (a plan built on crowded points has none and keeps
+        to the tiles); on the sweeps' own grids the plan's first set is,
         from 2^18 points on (2^17 in 2D), and further ones if that one crowded:
         other plans' re-pointing reads nothing back, so that a program whose
         points move need not wait for the device, and stays with the sweep."""
@@ -241,7 +250,7 @@ class _PointsND:
                 return E.sweep_load(self.pts)
         return None
 
-    def _uncrowded(self, load):
+    def _uncrowded(self, load, repoint=False):
         """Whether the sweep keeps the points. The sweeps' own grids are left
         only at a few times the tiles' time. Measured, us, sweep / tiles, radial
         points: 1e6 on 200 x 192 x 180, w = 6, spread 2738 / 460, gather
@@ -249,7 +258,7 @@ class _PointsND:
         1507 / 282."""
         slack = 1.0 if self._ext else (2.0 if self._ysweep else 3.0)
         load = load.item()  # 4 bytes, as the tile path's subproblem count
-        if not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack):
+        if not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack, repoint):
             return False
         # on extents the other route's sums are fp64 ones
         return (not self._ext or self.pts.kind != "zsweep"

@@ -188,16 +188,45 @@ def test_extents_no_less_precise_than_fp64_sums(eps, dens, most, mn):
 def test_extents_leave_dense_sets_to_fp64_sums(mn):
     """fp32 sums lose to the tiles' fp64 ones where a cell sums many points
     (7.7e-7 against 7.0e-7 at 20 a cell, w = 8), so from 8 a cell on the tiles
-    have them, on re-pointing as on a new plan."""
+    have them, on re-pointing as on a new plan; a plan built on them is one of
+    tiles for good, as it would build two point states for every set."""
     print("case extents dense", flush=True)
     rng = np.random.default_rng(37)
     N, cells = (45, 50, 55), 90 * 100 * 120
     thin, dense = _pts(rng, 6 * cells), _pts(rng, 12 * cells)
-    p = mn.Type1PlanND(dense, N, eps=1e-7)
-    assert p.pts.kind == "tiles" and p._store() is None
-    for x, kind in ((thin, "zsweep"), (dense, "tiles")):
+    for first, kinds in ((thin, ("tiles", "zsweep")), (dense, ("tiles", "tiles"))):
+        p = mn.Type1PlanND(first, N, eps=1e-7)
+        assert p.pts.kind == kinds[1]
+        for x, kind in zip((dense, thin), kinds):
+            p.set_sources(x)
+            assert p.pts.kind == kind and (p._store() is None) == (kind == "tiles")
+
+
+def test_repointing_weighs_both_point_states(mn):
+    """Moderately crowded sets, which the tiles would only just spread faster,
+    stay with the sweep on re-pointing: the step pays for the tiles' point
+    state too. Plans built on them take the tiles."""
+    print("case repoint setup", flush=True)
+    rng = np.random.default_rng(39)
+
+    def radial(M, dim):
+        v = rng.standard_normal((dim, M // 256 + 1, 1))
+        v = v / np.linalg.norm(v, axis=0) * np.linspace(-np.pi, np.pi, 256, endpoint=False)
+        return tuple(np.ascontiguousarray(a.reshape(-1)[:M]) for a in v)
+
+    for N, M, eps, sweep, later in (((1024, 1024), 300_000, 1e-6, "ymfma", "ymfma"),
+                                    ((45, 50, 55), 30_000, 1e-2, "zsweep", "tiles")):
+        x = radial(M, len(N))
+        p = mn.Type1PlanND(x, N, eps=eps)
+        assert p.pts.kind == "tiles"
         p.set_sources(x)
-        assert p.pts.kind == kind
+        assert p.pts.kind == later
+        p = mn.Type1PlanND(_pts(rng, M)[:len(N)], N, eps=eps)
+        p.set_sources(x)
+        assert p.pts.kind == sweep
+        c = _cplx(rng, M)
+        ref = mn.Type1PlanND(x, N, eps=eps, spread_method="gm").execute(c)
+        assert np.linalg.norm(p.execute(c) - ref) <= 3e-6 * np.linalg.norm(ref)
 
 
 @pytest.mark.parametrize("N,M,sweep", [((32, 32, 32), 1 << 18, "zsweep"),

@@ -583,7 +583,7 @@ def spread_ysweep(pts, beta, cs, grids):
                                      L.ptr(cs), L.ptr(grids), L.stream()), "spread_ysweep")
 
 
-def tiles_beat_ysweep(bins, w, n_up, P):
+def tiles_beat_ysweep(bins, w, P):
     """True when many points on a grid only the VALU y-sweep fits are better
     spread by the matrix-core tiles (bins: the tiles'): w = 7, us, sweep /
     tiles, 2e5 points on 256 x 270 412 / 34, 1e6 on 1024 x 900 194 / 63

@@ -104,9 +104,7 @@ class _PointsND:
         self._stream_interp = self._use_zstream and E.zstream_eligible(self.dim, self.w)
         if self._stream_interp:
             self.bins = E.make_bins(3, self.w, self.n_up, m=E.ZSTREAM_M)
-        elif self._cell_bytes == E.SPREAD_CELL_BYTES:
-            self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
-        else:
+        elif self._cell_bytes != E.SPREAD_CELL_BYTES:
             self.bins = E.make_bins(self.dim, self.w, self.n_up, cell_bytes=self._cell_bytes)
         self._zsweep = E.zsweep_eligible(self.dim, self.w, self.n_up) and self._zsweep_wanted()
         # grids off the sweep's blocks are stored with larger extents, at the
@@ -119,13 +117,9 @@ class _PointsND:
         # 2D: the y-window MFMA sweep where its geometry applies, else the
         # VALU y-sweep
         self._ymfma = self._use_zsweep and E.ymfma_eligible(self.dim, self.w, self.n_up)
-        self._ysweep = self._use_zsweep and (self._ymfma or
-                                             E.ysweep_eligible(self.dim, self.w, self.n_up))
-        if self._ysweep and not self._ymfma and E.tiles_beat_ysweep(self.bins, self.w, self.n_up,
-                                                                    self.P):
-            self._ysweep = False
-        if self._ysweep:
+        if self._use_zsweep and (self._ymfma or E.ysweep_eligible(self.dim, self.w, self.n_up)):
             self._ybins = E.make_bins(2, self.w, self.n_up, m=(16 if self._ymfma else 64, 1))
+        self._route_by_count()
         load = self._set_points(x64, building=True)
 
         # Mode deconvolution 1/phihat(2 pi k / n_up) on the uncentred fine grid
@@ -150,6 +144,16 @@ class _PointsND:
                 self._watch = True
             self.pts = None
             self._set_points(x64, tiles=True)
+
+    _ybins = None
+
+    def _route_by_count(self):
+        """What depends on the number of points: the tiles of a spread, and
+        whether they take many points over from the VALU y-sweep."""
+        if self._cell_bytes == E.SPREAD_CELL_BYTES:
+            self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
+        self._ysweep = self._ybins is not None and (
+            self._ymfma or not E.tiles_beat_ysweep(self.bins, self.w, self.P))
 
     # the z-sweep point state is built in the spread's key order unless set
     _zgather_points = False
@@ -440,6 +444,7 @@ class Type1PlanND(_PointsND):
         if P < 1 or not all(v.numel() == P for v in x64):
             raise ValueError("coordinate arrays must be non-empty, equal length")
         self.P = P
+        self._route_by_count()
         if not (isinstance(self.pts, (E.ZSweepPoints, E.YSweepPoints)) and self.pts.P == P):
             self.pts = None  # nothing to reuse: free the old point state first
         self._set_points(x64)

@@ -271,3 +271,23 @@ def test_native_route_depends_on_first_and_current_set_only(N, M, sweep, mn):
             torch.cuda.set_sync_debug_mode("default")
         assert p.pts.kind == sweep
         check(p, "crowd")
+
+
+def test_route_follows_number_of_points(mn):
+    """Re-pointing to another number of points takes the tiles and the route of
+    a plan built on so many: the VALU y-sweep's grids go to the tiles from 2^17
+    points on, the tiles' bins follow the points per cell."""
+    print("case route by count", flush=True)
+    rng = np.random.default_rng(40)
+    pts = lambda M: tuple(rng.uniform(-np.pi, np.pi, M) for _ in range(2))
+    for N, sizes, kinds in (((128, 135), (2000, 1 << 17, 2000), ("ysweep", "tiles", "ysweep")),
+                            ((125, 135), (2000, 60000, 2000), ("tiles",) * 3)):
+        p = mn.Type1PlanND(pts(sizes[-1]), N, eps=1e-6)
+        for M, kind in zip(sizes, kinds):
+            x, c = pts(M), _cplx(rng, M)
+            p.set_sources(x)
+            q = mn.Type1PlanND(x, N, eps=1e-6)
+            assert p.pts.kind == q.pts.kind == kind
+            assert list(p.pts.bins.m) == list(q.pts.bins.m)
+            ref = q.execute(c)
+            assert np.linalg.norm(p.execute(c) - ref) <= 1e-6 * np.linalg.norm(ref)

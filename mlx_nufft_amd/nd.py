@@ -149,11 +149,13 @@ class _PointsND:
 
     def _route_by_count(self):
         """What depends on the number of points: the tiles of a spread, and
-        whether they take many points over from the VALU y-sweep."""
+        whether they take many points over from the VALU y-sweep (not under
+        stream capture, where their subproblem count cannot be read back)."""
         if self._cell_bytes == E.SPREAD_CELL_BYTES:
             self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
         self._ysweep = self._ybins is not None and (
-            self._ymfma or not E.tiles_beat_ysweep(self.bins, self.w, self.P))
+            self._ymfma or not E.tiles_beat_ysweep(self.bins, self.w, self.P)
+            or torch.cuda.is_current_stream_capturing())
 
     # the z-sweep point state is built in the spread's key order unless set
     _zgather_points = False
@@ -231,7 +233,9 @@ class _PointsND:
         to the tiles); on the sweeps' own grids the plan's first set is,
         from 2^18 points on (2^17 in 2D), and further ones if that one crowded:
         other plans' re-pointing reads nothing back, so that a program whose
-        points move need not wait for the device, and stays with the sweep."""
+        points move need not wait for the device, and stays with the sweep.
+        Under stream capture, where nothing can be read, the sweep has every
+        set."""
         prec64 = self.prec == "crit64"
         with tm("setpts+sort+tables"):
             prev = getattr(self, "pts", None)
@@ -250,7 +254,8 @@ class _PointsND:
             del prev
             many = self._ymfma if self._ysweep else True
             many = many and self.P >= 1 << (17 if self._ysweep else 18)
-            if self._ext or ((building or self._watch) and many):
+            look = self._ext or ((building or self._watch) and many)
+            if look and not torch.cuda.is_current_stream_capturing():
                 return E.sweep_load(self.pts)
         return None
 

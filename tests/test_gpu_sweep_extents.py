@@ -291,3 +291,36 @@ def test_route_follows_number_of_points(mn):
             assert list(p.pts.bins.m) == list(q.pts.bins.m)
             ref = q.execute(c)
             assert np.linalg.norm(p.execute(c) - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("N,M,crowded,kind", [((128, 135), 1 << 17, False, "ysweep"),
+                                              ((128, 128), 1 << 17, True, "ymfma"),
+                                              ((32, 32, 32), 1 << 18, True, "zsweep"),
+                                              ((27, 25, 33), 20000, False, "zsweep")])
+def test_step_under_capture(N, M, crowded, kind, mn):
+    """A step (set_sources and execute) captured into a graph: nothing can be
+    read back there, so the sweep takes the set where the grid has one; every
+    replay equals the eager tiles, with eager work in between."""
+    print(f"case capture N={N}", flush=True)
+    rng = np.random.default_rng(41)
+    dim = len(N)
+    wide = [[rng.uniform(-np.pi, np.pi, M) for _ in range(dim)] for _ in range(3)]
+    first = [rng.uniform(0.1, 0.2, M) for _ in range(dim)] if crowded else wide[0]
+    x = [torch.from_numpy(v.copy()).cuda() for v in wide[0]]
+    c = torch.from_numpy(_cplx(rng, M)).cuda()
+    p = mn.Type1PlanND([torch.from_numpy(v).cuda() for v in first], N, eps=1e-6)
+    p.set_sources(x)
+    p.execute(c, return_np=False)       # tables and buffers
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        p.set_sources(x)
+        out = p.execute(c, return_np=False)
+    assert p.pts.kind == kind
+    for w in wide:
+        for d in range(dim):
+            x[d].copy_(torch.from_numpy(w[d]))
+        graph.replay()
+        got = out.cpu().numpy()
+        ref = mn.Type1PlanND(tuple(w), N, eps=1e-6, spread_method="gm").execute(c)
+        assert np.linalg.norm(got - ref) <= 3e-6 * np.linalg.norm(ref)

@@ -154,7 +154,8 @@ class _PointsND:
         if self._cell_bytes == E.SPREAD_CELL_BYTES:
             self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
         self._ysweep = self._ybins is not None and (
-            self._ymfma or not E.tiles_beat_ysweep(self.bins, self.w, self.P)
+            self._ymfma or self.spread_method == "od"
+            or not E.tiles_beat_ysweep(self.bins, self.w, self.P)
             or torch.cuda.is_current_stream_capturing())
 
     # the z-sweep point state is built in the spread's key order unless set
@@ -254,6 +255,7 @@ class _PointsND:
             del prev
             many = self._ymfma if self._ysweep else True
             many = many and self.P >= 1 << (17 if self._ysweep else 18)
+            many = many and (self._zgather_points or self.spread_method != "od")
             look = self._ext or ((building or self._watch) and many)
             if look and not torch.cuda.is_current_stream_capturing():
                 return E.sweep_load(self.pts)
@@ -339,12 +341,15 @@ class Type1PlanND(_PointsND):
 
     def __init__(self, x, n_modes, eps=1e-6, isign=+1, upsampfac=2.0, prec="crit64",
                  sort_points=True, spread_method="auto"):
-        """spread_method: "auto" picks the fastest spread for the geometry
-        (3D: the owner-computes z-sweep; 2D: the y-sweep; else LDS tiles);
-        "od" does the same but first raises ValueError where the reference's
-        output-driven spread would not apply; "gm" forces the LDS-tile
-        spread with its atomic flush, this engine's counterpart of the
-        reference's global-memory atomic spread (ref: nd.py:397-404)."""
+        """spread_method: "auto" picks the fastest spread for the grid
+        and the points (3D: the owner-computes z-sweep; 2D: the y-sweep;
+        where points crowd or the grid does not fit them, tiles); "od" first
+        raises ValueError where the reference's output-driven spread would not
+        apply and keeps the sweeps on their own grids whatever the points, so
+        that results repeat bit for bit there; "gm" forces the tiles, this
+        engine's counterpart of the reference's global-memory atomic spread
+        (ref: nd.py:397-404). Tiles add their edges with atomics, in an order
+        that varies from run to run."""
         if spread_method not in SPREAD_METHODS:
             raise PlanArgumentError(f"spread_method must be one of {SPREAD_METHODS}, got "
                                     f"{spread_method!r}")

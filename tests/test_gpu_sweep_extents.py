@@ -324,3 +324,21 @@ def test_step_under_capture(N, M, crowded, kind, mn):
         got = out.cpu().numpy()
         ref = mn.Type1PlanND(tuple(w), N, eps=1e-6, spread_method="gm").execute(c)
         assert np.linalg.norm(got - ref) <= 3e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("N,M,kind", [((32, 32, 32), 1 << 18, "zsweep"),
+                                      ((128, 128), 1 << 17, "ymfma"),
+                                      ((128, 135), 1 << 17, "ysweep")])
+def test_od_keeps_the_sweep(N, M, kind, mn):
+    """spread_method="od" keeps crowded and dense sets on the owner-computes
+    sweeps, whose results repeat bit for bit."""
+    print(f"case od N={N}", flush=True)
+    rng = np.random.default_rng(42)
+    x = tuple(rng.uniform(0.1, 0.2, M) for _ in N)
+    c = _cplx(rng, M)
+    p = mn.Type1PlanND(x, N, eps=1e-6, spread_method="od")
+    assert p.pts.kind == kind and mn.Type1PlanND(x, N, eps=1e-6).pts.kind == "tiles"
+    one = p.execute(c)
+    assert np.array_equal(p.execute(c), one)
+    p.set_sources(x)
+    assert p.pts.kind == kind and np.array_equal(p.execute(c), one)

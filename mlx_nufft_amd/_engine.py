@@ -315,8 +315,10 @@ def sweep_load(pts):
 
 
 # points a us of one sweep wave, and us the tile kernels, which split crowded
-# bins, take for 1000 points per unit of w
-_SWEEP_RATES = {"zsweep": (20.0, 0.04), "zgather": (8.0, 0.017), "ymfma": (21.0, 0.012)}
+# bins, take for 1000 points per unit of w. On radial points a y-window wave does
+# 51 to 53; the 3D ones 25 to 28 and 14 to 18, put lower here: so the tiles were
+# faster, or 5 us slower at most, in every set handed over (3e4 to 5e6 points).
+_SWEEP_RATES = {"zsweep": (20.0, 0.04), "zgather": (8.0, 0.017), "ymfma": (52.0, 0.012)}
 
 
 def sweep_balanced(load, kind, w, P, slack=1.0, repoint=False):

@@ -262,12 +262,13 @@ class _PointsND:
         return None
 
     def _uncrowded(self, load, repoint=False):
-        """Whether the sweep keeps the points. The sweeps' own grids are left
-        only at a few times the tiles' time. Measured, us, sweep / tiles, radial
-        points: 1e6 on 200 x 192 x 180, w = 6, spread 2738 / 460, gather
-        2625 / 135; 2D, w = 7, 1e6 on 1024^2 455 / 90, 5e6 on 2048^2
-        1507 / 282."""
-        slack = 1.0 if self._ext else (2.0 if self._ysweep else 3.0)
+        """Whether the sweep keeps the points. The sweeps' own 3D grids are
+        left only at a few times the tiles' time, 2D ones, whose estimate leaves
+        out the tiles' zero fill, at a little more. Measured, us, sweep / tiles,
+        radial points: 1e6 on 200 x 192 x 180, w = 6, spread 2738 / 460, gather
+        2625 / 135; 2D with the transform, w = 7, 131072 on 2048^2 99 / 125
+        (kept), 3e5 153 / 130, 1e6 on 1024^2 472 / 100."""
+        slack = 1.0 if self._ext else (1.2 if self._ysweep else 3.0)
         load = load.item()  # 4 bytes, as the tile path's subproblem count
         if not E.sweep_balanced(load, self.pts.kind, self.w, self.P, slack, repoint):
             return False

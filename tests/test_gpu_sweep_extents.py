@@ -342,3 +342,16 @@ def test_od_keeps_the_sweep(N, M, kind, mn):
     assert np.array_equal(p.execute(c), one)
     p.set_sources(x)
     assert p.pts.kind == kind and np.array_equal(p.execute(c), one)
+
+
+def test_crowding_rule_2d_near_break_even(mn):
+    """Radial points on 2048^2, w = 7: 2^17 stay with the sweep (99 us against
+    125 with the tiles), 3e5 leave it (153 against 130)."""
+    print("case crowding rule 2d", flush=True)
+    rng = np.random.default_rng(43)
+    for M, kind in ((1 << 17, "ymfma"), (300_000, "tiles")):
+        per = int(np.sqrt(M))
+        v = rng.standard_normal((2, M // per + 1, 1))
+        v = v / np.linalg.norm(v, axis=0) * np.linspace(-np.pi, np.pi, per, endpoint=False)
+        x = tuple(np.ascontiguousarray(a.reshape(-1)[:M]) for a in v)
+        assert mn.Type1PlanND(x, (1024, 1024), eps=1e-6).pts.kind == kind

@@ -103,14 +103,22 @@ def spread_bins(dim, w, n_up, P):
     and 2D from w = 5 where the points fill the grid (2000^2, w = 6: 0.3
     points per cell 90 / 101, 0.6 143 / 101, 2.4 506 / 281; w = 12: 0.3
     272 / 387, 0.6 505 / 408); wider 2D kernels leave bins of 4 cells or fewer
-    and need more. MN_BIN_M overrides the bins."""
+    and need more. 3D kernels of 13 to 16 cells leave bins of 4 to 1, which are
+    still the faster ones (120^3, 3e4 to 3e6 points: w = 13 1775 / 478 to
+    12669 / 1337, w = 16 6704 / 1112 to 65124 / 55538), until there are so many
+    of them that a launch of 256 threads for each that holds points would pass
+    2^32, or their tables (24 bytes a bin) 3 GB. MN_BIN_M overrides the bins."""
     if dim == 1 or w <= 4 or os.environ.get("MN_BIN_M"):
         return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
     if dim == 2:
         full = 0.4 if w <= 12 else 1.0
         if w > 14 or P < full * float(n_up[0]) * float(n_up[1]):
             return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
-    return make_bins(dim, w, n_up, m=[max(1, min(17 - w, int(k))) for k in n_up])
+    bins = make_bins(dim, w, n_up, m=[max(1, min(17 - w, int(k))) for k in n_up])
+    # subproblems: one for each bin with points, and one more for every 1024
+    if bins.nbins > 1 << 27 or min(bins.nbins, P) + P // MSUB + MSUB >= 1 << 24:
+        return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
+    return bins
 
 
 def spread_msub(bins, P):

@@ -333,3 +333,21 @@ def test_bench_refuses_more_than_one_gpu():
     assert r.returncode == 2
     assert "one GPU only" in r.stderr
     assert r.stdout.strip() == ""
+
+
+@pytest.mark.parametrize("n,w,P,m", [(512, 16, 20_000_000, 2), (512, 16, 1_000_000, 1),
+                                     (1250, 16, 1_000_000, 2), (512, 15, 100_000_000, 3),
+                                     (256, 16, 10_000_000, 1), (512, 7, 20_000_000, 10)])
+def test_spread_bins_stay_launchable(clib, monkeypatch, n, w, P, m):
+    """Bins of the 3D tile spread: 17 - w cells, or 18 - w where there would be
+    more subproblems than a launch of 256 threads for each can hold, or more
+    bins than are accepted."""
+    from mlx_nufft_amd import _engine as E
+
+    monkeypatch.setattr(E, "_budget", E.TILE_BUDGET)
+    bins = E.spread_bins(3, w, [n] * 3, P)
+    assert list(bins.m) == [m] * 3
+    assert clib.mn_subproblem_workspace_bytes(ctypes.byref(bins)) > 0
+    # bins that hold any of P uniform points, and the further subproblems
+    nsub = -bins.nbins * np.expm1(-P / bins.nbins) + P // E.spread_msub(bins, P)
+    assert 256 * nsub < 1 << 32

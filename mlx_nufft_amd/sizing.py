@@ -81,7 +81,6 @@ def _quadrature(beta, w, nquad):
     t, wt = _GL[nquad]
     dq = 0.5 * (t + 1.0) * (w / 2.0)
     fq = wt * (w / 4.0) * es_kernel(dq, beta, w)
-    dq.flags.writeable = fq.flags.writeable = False  # shared by every caller
     return dq, fq
 
 
@@ -91,7 +90,8 @@ def quadrature(beta, w, nquad=128):
 
     ref: sizing.py:74-85 (128-point Gauss-Legendre on [0, w/2]).
     """
-    return _quadrature(float(beta), int(w), int(nquad))
+    dq, fq = _quadrature(float(beta), int(w), int(nquad))
+    return dq.copy(), fq.copy()  # the cached pair is shared
 
 
 def kernel_ft(xi, beta, w, nquad=128):

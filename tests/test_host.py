@@ -351,3 +351,15 @@ def test_spread_bins_stay_launchable(clib, monkeypatch, n, w, P, m):
     # bins that hold any of P uniform points, and the further subproblems
     nsub = -bins.nbins * np.expm1(-P / bins.nbins) + P // E.spread_msub(bins, P)
     assert 256 * nsub < 1 << 32
+
+
+def test_quadrature_arrays_are_the_callers():
+    """Every call returns arrays of its own that may be written to."""
+    from mlx_nufft_amd.sizing import quadrature
+
+    a = quadrature(16.1, 7)
+    b = [v.copy() for v in a]
+    for v in a:
+        v[:] = -1.0
+    for v, r in zip(quadrature(16.1, 7), b):
+        assert np.array_equal(v, r)

@@ -363,3 +363,19 @@ def test_quadrature_arrays_are_the_callers():
         v[:] = -1.0
     for v, r in zip(quadrature(16.1, 7), b):
         assert np.array_equal(v, r)
+
+
+def test_plan_decs_are_evaluated_once():
+    """The fp64 factors of a plan are one list, which a program may also set."""
+    from mlx_nufft_amd import sizing
+    from mlx_nufft_amd.nd import Type1PlanND
+
+    p = object.__new__(Type1PlanND)
+    p.N, p.n_up = (9, 4), [18, 14]
+    p.w, p.beta = sizing.kernel_params(1e-6, 2.0)
+    for v, n, N in zip(p.decs, p.n_up, p.N):
+        k = np.arange(-(N // 2), N - N // 2)
+        assert np.allclose(v * sizing.kernel_ft(2 * np.pi * k / n, p.beta, p.w), 1.0)
+    assert p.decs is p.decs
+    p.decs = [np.ones(9), np.ones(4)]
+    assert p.decs[1].sum() == 4.0

@@ -578,8 +578,8 @@ int mn_pad_deconv_fft(int dim, const int64_t n_up[3], const int64_t N[3], int64_
                       int64_t work_bytes, void *grid, mn_stream_t stream);
 /*
  * The same two transforms for fine grids of any size 2^a 3^b 5^c
- * (mn_fftg_supported: axes of at least 4 and, split, up to 2048^2, longer ones than 2048 split into two
- * passes). ext gives the extents the grid is stored with (NULL: n_up);
+ * (mn_fftg_supported: axes of 4 to 2048, and up to 2048^2 where such an axis
+ * splits into two passes). ext gives the extents the grid is stored with (NULL: n_up);
  * ext[d] in [n_up[d], 2 n_up[d]], larger ones in 2D and 3D only and with a
  * last axis of at most 2048. Type 1 adds the cells at x + n_up[d] < ext[d]
  * to cell x before it transforms; type 2 stores every cell at all its images

@@ -607,10 +607,11 @@ def ymfma_segment(n_up):
     """y-segment per wavefront of the y-window MFMA sweep: the one (8 to 256
     cells) that minimises rounds x (yseg + 8), as zsweep_segment, for one wave
     per block (up to 8 vectors), so that a batch sums as its vectors do alone.
-    Measured, us,
-    the chosen length and the 32 cells that used to be the least: 1e5 points on
-    256^2, w = 7 (8) 21 and 35, 8 vectors 61 and 117; 1e6 on 512^2 (16) 53 and
-    74; 1e7 on 2048^2, 8 vectors (128) 935, 969 at 64."""
+    Measured, us, w = 7, one vector / 8, at the chosen length and at 32 cells:
+    1e5 points on 256^2 (8) 19 / 57 and 34 / 108; 1e6 on 512^2 (8) 51 / 178 and
+    72 / 250; 1e7 on 2048^2 (128) 265 / 940 and 324 / 1036 (327 / 974 at 64).
+    Sets that crowd like longer segments less: 1e7 radial points there 16 %
+    slower than at 64."""
     blocks = n_up[0] // 16
 
     def cost(y):

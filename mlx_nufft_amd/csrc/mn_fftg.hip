@@ -143,7 +143,8 @@ bool fg_split(int64_t n, int64_t *n1, int64_t *n2) {
 
 bool fg_axis_ok(int64_t n) {
     int64_t a, b;
-    return n >= 4 && n <= FG_SPLIT * FG_SPLIT && (n <= FG_SPLIT ? fg_find(n) != nullptr : fg_split(n, &a, &b));
+    return n >= 4 && n <= FG_SPLIT * FG_SPLIT &&
+           (n <= FG_SPLIT ? fg_find(n) != nullptr : fg_split(n, &a, &b));
 }
 
 struct FgPlan {

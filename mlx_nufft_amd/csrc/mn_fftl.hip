@@ -32,7 +32,7 @@
 // keep a part of its lines and of their outputs: it transforms lines
 // q * period + r with q and r in given ranges and stores outputs [r0, r0 + nr).
 // Skipped cells are neither written nor read. At 640^3 (486^3 values in,
-// middle 536 kept) the passes move 11.4 instead of 15.1 GB; kept ranges of whole
+// middle 528 kept) the passes move 11.4 instead of 15.1 GB; kept ranges of whole
 // multiples of 16 also give odd lengths tiles of several lines.
 //
 // ref: gpu_t3.py:630-651 (t3pad: pad + mode deconvolution), gpu_t3.py:94-148
@@ -471,7 +471,8 @@ __global__ void k_fl_twiddles(double2 *tw, int n, int S) {
 
 // Radices for n = 2^a 3^b 5^c: as few stages as the radices allow, then the
 // smallest ones. Odd ones go first: the first stage's stores are its radix
-// apart, and even strides share LDS banks. 0 if n has another factor or needs more than FL_MAXST stages.
+// apart, and even strides share LDS banks. 0 if n has another factor or needs
+// more than FL_MAXST stages.
 int fl_radices(int64_t n, int *rad, int most = FL_MAXST, int top = 12, bool six = true) {
     if (n == 1) return 0;
     int best = 0, sum = 0, cur[FL_MAXST];

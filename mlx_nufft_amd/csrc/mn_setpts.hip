@@ -88,7 +88,8 @@ constexpr int ZP_THREADS = 256;
 constexpr int ZP_ITEMS = 4;
 template <bool GATHER>
 __global__ __launch_bounds__(ZP_THREADS) void k_zs_setpts(int64_t P, D3 x, int n0, int n1, int n2,
-                                                          int e1, int e2, int w, double h0, double h1, double h2,
+                                                          int e1, int e2, int w, double h0,
+                                                          double h1, double h2,
                                                           int prec64, uint32_t *__restrict__ word,
                                                           F3 fro) {
     const int64_t j0 = (int64_t)blockIdx.x * (ZP_THREADS * ZP_ITEMS) + threadIdx.x;
@@ -316,8 +317,8 @@ int mn_setpts_t12(const mn_bins *g, int64_t P, const double *const x[3], int pre
     return MN_OK;
 }
 
-static int zs_setpts(bool gather, const mn_bins *g, const int64_t n[3], int64_t P, const double *const x[3],
-                     int prec64, uint32_t *word, float *const fr[3], mn_stream_t stream) {
+static int zs_setpts(bool gather, const mn_bins *g, const int64_t n[3], int64_t P,
+                     const double *const x[3], int prec64, uint32_t *word, float *const fr[3], mn_stream_t stream) {
     clear_error();
     int rc = zsweep_check(g);
     if (rc) return rc;
@@ -334,7 +335,8 @@ static int zs_setpts(bool gather, const mn_bins *g, const int64_t n[3], int64_t 
     }
     auto kern = gather ? k_zs_setpts<true> : k_zs_setpts<false>;
     kern<<<blocks_for(P, ZP_THREADS * ZP_ITEMS), ZP_THREADS, 0, as_stream(stream)>>>(
-        P, xs, (int)n[0], (int)n[1], (int)n[2], (int)g->n[1], (int)g->n[2], g->w, h[0], h[1], h[2], prec64, word, fo);
+        P, xs, (int)n[0], (int)n[1], (int)n[2], (int)g->n[1], (int)g->n[2], g->w, h[0], h[1],
+        h[2], prec64, word, fo);
     MN_LAUNCH_CHECK("zsweep_setpts");
     return MN_OK;
 }

@@ -235,10 +235,9 @@ __global__ __launch_bounds__(256) void k_spread_tiled(Geom g, float bl2e, float 
     }
 }
 
-// 3D fp64 tile spread on the matrix cores (type-3 sources, complex128 grid),
-// for padded tiles of at most 16 cells per dim. Instead of one LDS
-// atomic per tap, the tile is accumulated by v_mfma_f64_16x16x4f64 outer
-// products: for each x plane of the tile, D[y][z] += sum over 4 points k of
+// 3D tile spread on the matrix cores, products and sums in fp64, for padded
+// tiles of at most 16 cells per dim. Instead of one LDS atomic per tap, the
+// tile is accumulated by v_mfma_f64_16x16x4f64 outer products: for each x plane of the tile, D[y][z] += sum over 4 points k of
 // A[y][k] B[k][z] with A = wx(x) wy(y) (exact in fp64: the weights are fp32)
 // and B = c_k wz(z) (the strength times its prephase, fp64, as the
 // LDS-atomic kernel forms it); the real and imaginary planes are two MFMAs
@@ -251,14 +250,13 @@ __global__ __launch_bounds__(256) void k_spread_tiled(Geom g, float bl2e, float 
 // points, skipping the MFMAs of a plane that none of the 4 points reaches
 // (the subproblem is taken in x-footprint order, so neighbouring points
 // share planes). After the last batch the accumulators are flushed to the
-// grid with fp64 atomics, re and im of a cell from adjacent lanes, skipping
-// zeros. Only the summation order differs from the LDS-atomic kernel.
+// grid with atomics of its own type, re and im of a cell from adjacent lanes,
+// skipping zeros. Only the summation order differs from the LDS-atomic kernel.
 // (Tiles of 32 x 16 x 16 cells with eight waves, bins of 33 - w along x,
 // measured 5 % slower at cfg 5: 0.477 against 0.456 ms.)
 typedef double mn_v4d __attribute__((ext_vector_type(4)));
 constexpr int MN_SUB_MAX_ORDER = 1024;  // points per subproblem the x-order takes
 
-//
 // Real is the grid's component type: double for type-3 sources, float for the
 // types 1 and 2, whose vectors blockIdx.y walks (strides cstride and gstride).
 // With a float grid, 2e6 points and w = 7 on 270 x 240 x 180 take 0.56 ms

@@ -9,10 +9,10 @@ with k_d in [-(N_d//2), (N_d-1)//2] (modeord=0, even or odd N_d) and any x
 the transform; all device work is HIP kernels behind the C-ABI.
 
 Pipeline (type 1): fp64 setpts (fold, rescale, cell/frac, sort key) ->
-stable radix sort carrying the point data -> ES spread (3D: owner-computes
-z-sweep, no atomics; otherwise LDS tiles flushed with atomics) -> FFT with
-the mode crop and deconvolution fused (pruned per-axis FFT on power-of-two
-grids, else rocFFT + crop). Type 2 runs the adjoint chain: deconvolve +
+stable radix sort carrying the point data -> ES spread (3D and 2D:
+owner-computes sweeps, no atomics; where they do not apply or points crowd,
+tiles flushed with atomics) -> FFT with the mode crop and deconvolution fused
+(pruned per-axis FFTs for 5-smooth grids, else rocFFT + crop). Type 2 runs the adjoint chain: deconvolve +
 zero-pad + FFT -> LDS-tiled interpolation written straight to caller order.
 """
 

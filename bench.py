@@ -108,6 +108,16 @@ def cpu_baseline(x, c, N, eps):
             "seconds": {k: round(v, 4) for k, v in parts.items()}}
 
 
+def spread_kernel_name(plan):
+    """The kernel that a plan's single-vector 3D spread launches, as a profiler
+    names it."""
+    if plan.pts.kind == "zsweep":
+        return f"k_spread_zsweep<{plan.w}, false, 1, {'true' if plan.pts.ext else 'false'}>"
+    if max(plan.bins.m) + plan.w - 1 <= 16:
+        return f"k_spread_tile_mfma<{plan.w}, float>"
+    return f"k_spread_tiled<3, {plan.w}, false, false>"
+
+
 def spread_traffic(kernel):
     """HBM bytes per spread launch (FETCH_SIZE + WRITE_SIZE, calibrated) from
     the committed rocprofv3 summary, with its provenance. The summary records
@@ -390,8 +400,7 @@ def main():
     fk = plan.execute(cd, return_np=False)
     plan_w, plan_bins = plan.w, [plan.bins.m[d] for d in range(3)]
     zsweep = plan.pts.kind == "zsweep"
-    spread_kernel = (f"k_spread_zsweep<{plan_w}, false, 1>" if zsweep
-                     else f"k_spread_tiled<3,{plan_w},false>")
+    spread_kernel = spread_kernel_name(plan)
     traffic, traffic_src = spread_traffic(spread_kernel)
     del plan
     p2 = mn.Type2PlanND(tuple(xd), N, eps=eps, isign=-1)

@@ -379,3 +379,22 @@ def test_plan_decs_are_evaluated_once():
     assert p.decs is p.decs
     p.decs = [np.ones(9), np.ones(4)]
     assert p.decs[1].sum() == 4.0
+
+
+@pytest.mark.parametrize("w,kind,m,ext", [(6, "zsweep", 8, False), (7, "zsweep", 8, True),
+                                          (6, "tiles", 11, False), (4, "tiles", 14, False)])
+def test_bench_names_a_kernel_that_exists(clib, w, kind, m, ext):
+    """The spread kernel that bench.py reports, and whose traffic it looks up,
+    is one of the library's."""
+    import subprocess
+    import types
+
+    from mlx_nufft_amd import _lib
+    import bench
+
+    plan = types.SimpleNamespace(w=w, bins=types.SimpleNamespace(m=[m] * 3),
+                                 pts=types.SimpleNamespace(kind=kind, ext=ext))
+    name = bench.spread_kernel_name(plan)
+    out = subprocess.run(["nm", "-C", str(_lib.LIB_PATH)], capture_output=True, text=True,
+                         check=True, timeout=120).stdout
+    assert f"{name}(" in out

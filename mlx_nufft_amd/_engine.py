@@ -121,16 +121,20 @@ def spread_bins(dim, w, n_up, P):
     return bins
 
 
-def spread_msub(bins, P):
+def spread_msub(bins, P, sigma=2.0):
     """Points per subproblem of the type-1 tile spread: MSUB, but in steps of
     the matrix-core kernels' 64-point batches fewer where MSUB would leave the
     chip idle (2D tiles take one wave, 3D ones four): 1e4 points on
     18 x 24 x 30, w = 7, take 27 us instead of 100, 5e5 on 66 x 74 36 instead
     of 50; 5e5 points on 144 x 128 x 125 already fill it (more, smaller ones
     flush more tiles: 585 against 527 us for 4 vectors). The LDS kernels keep
-    MSUB (1e5 points in 1D: 17 us, 19 to 25 with fewer)."""
+    MSUB (1e5 points in 1D: 17 us, 19 to 25 with fewer), and so does sigma < 2,
+    whose deconvolution magnifies the rounding of the fp32 sums that join the
+    subproblems: w = 9 at sigma = 1.25 on 18 x 30 x 24, 9e3 / 1e5 points, 9.2e-6
+    / 1.22e-5 from 64 bits with short ones, 6.7e-6 / 8.1e-6 with MSUB and 7.3e-6
+    / 9.1e-6 in LDS tiles (47 / 76, 71 / 148 and 188 / 333 us)."""
     dim, w = bins.dim, bins.w
-    if dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
+    if sigma < 2.0 or dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
         return MSUB
     return max(64, min(MSUB, (P // (2048 if dim == 2 else 512) + 63) // 64 * 64))
 
@@ -510,10 +514,11 @@ class GroupSplit:
     non-empty groups and builds the subset's start table just before it is
     used: z-/y-sweep key starts in one shared buffer (rebuilt in stream
     order, after the previous group's spread has read it), or the tile
-    spread's subproblem table."""
+    spread's subproblem table (sigma: spread_msub)."""
 
-    def __init__(self, pts, glabel, G):
+    def __init__(self, pts, glabel, G, sigma=2.0):
         self.pts = pts
+        self.sigma = sigma
         self.G = G
         dim = pts.bins.dim
         gs = glabel[pts.perm.long()]
@@ -541,7 +546,8 @@ class GroupSplit:
             if pts.kind == "tiles":
                 sub = _Subset("tiles", pts.bins, e - s, perm=c[1][s:e], skey=c[0][s:e], frs=frs,
                               i1s=[r[s:e] for r in c[2 + dim:2 + 2 * dim]])
-                sub.info, sub.nsub = build_subproblems(pts.bins, sub.skey, spread_msub(pts.bins, sub.P))
+                sub.info, sub.nsub = build_subproblems(
+                    pts.bins, sub.skey, spread_msub(pts.bins, sub.P, self.sigma))
                 yield g, sub
                 continue
             if self._startbuf is None:

@@ -361,7 +361,7 @@ class Type1PlanND(_PointsND):
         super().__init__(x, n_modes, eps, isign, upsampfac, prec, sort_points)
 
     def _msub(self):
-        return E.spread_msub(self.bins, self.P)
+        return E.spread_msub(self.bins, self.P, self.sigma)
 
     def _strengths(self, c):
         cd = L.to_dev_c64(c, self.device).reshape(-1)
@@ -482,7 +482,7 @@ class Type1PlanND(_PointsND):
         G = int(gl.max()) + 1 if gl.numel() else 0
         out = torch.zeros((max(G, 0), *self.N), dtype=torch.complex64, device=self.device)
         if G > 0:
-            split = E.GroupSplit(self.pts, gl, G)
+            split = E.GroupSplit(self.pts, gl, G, self.sigma)
             del gl
             grid = self._fine_grid(1)
             tm = self._timer()

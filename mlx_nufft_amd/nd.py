@@ -147,17 +147,22 @@ class _PointsND:
             self._set_points(x64, tiles=True)
 
     _ybins = None
+    _routed = None
 
     def _route_by_count(self):
         """What depends on the number of points: the tiles of a spread, and
         whether they take many points over from the VALU y-sweep (not under
         stream capture, where their subproblem count cannot be read back)."""
+        valu = self._ybins is not None and not self._ymfma
+        key = (self.P, valu and torch.cuda.is_current_stream_capturing())
+        if key == self._routed:
+            return
+        self._routed = key
         if self._cell_bytes == E.SPREAD_CELL_BYTES:
             self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
         self._ysweep = self._ybins is not None and (
             self._ymfma or self.spread_method == "od"
-            or not E.tiles_beat_ysweep(self.bins, self.w, self.P)
-            or torch.cuda.is_current_stream_capturing())
+            or not E.tiles_beat_ysweep(self.bins, self.w, self.P) or key[1])
 
     # the z-sweep point state is built in the spread's key order unless set
     _zgather_points = False

@@ -128,13 +128,14 @@ def spread_msub(bins, P, sigma=2.0):
     18 x 24 x 30, w = 7, take 27 us instead of 100, 5e5 on 66 x 74 36 instead
     of 50; 5e5 points on 144 x 128 x 125 already fill it (more, smaller ones
     flush more tiles: 585 against 527 us for 4 vectors). The LDS kernels keep
-    MSUB (1e5 points in 1D: 17 us, 19 to 25 with fewer), and so does sigma < 2,
-    whose deconvolution magnifies the rounding of the fp32 sums that join the
-    subproblems: w = 9 at sigma = 1.25 on 18 x 30 x 24, 9e3 / 1e5 points, 9.2e-6
-    / 1.22e-5 from 64 bits with short ones, 6.7e-6 / 8.1e-6 with MSUB and 7.3e-6
-    / 9.1e-6 in LDS tiles (47 / 76, 71 / 148 and 188 / 333 us)."""
+    MSUB (1e5 points in 1D: 17 us, 19 to 25 with fewer), and so does sigma < 2
+    from w = 8 on, whose deconvolution magnifies the rounding of the fp32 sums
+    that join the subproblems: w = 9 at sigma = 1.25 on 18 x 30 x 24, 9e3 / 1e5
+    points, 9.2e-6 / 1.22e-5 from 64 bits with short ones, 6.7e-6 / 8.1e-6 with
+    MSUB and 7.3e-6 / 9.1e-6 in LDS tiles (47 / 76, 71 / 148 and 188 / 333 us);
+    at w = 7 the kernel's own 9.9e-5 hides it."""
     dim, w = bins.dim, bins.w
-    if sigma < 2.0 or dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
+    if (sigma < 2.0 and w >= 8) or dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
         return MSUB
     return max(64, min(MSUB, (P // (2048 if dim == 2 else 512) + 63) // 64 * 64))
 

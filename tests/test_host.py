@@ -398,3 +398,12 @@ def test_bench_names_a_kernel_that_exists(clib, w, kind, m, ext):
     out = subprocess.run(["nm", "-C", str(_lib.LIB_PATH)], capture_output=True, text=True,
                          check=True, timeout=120).stdout
     assert f"{name}(" in out
+
+
+def test_subproblem_size_follows_sigma(clib, monkeypatch):
+    """Short subproblems only where the rounding of their joining does not show."""
+    from mlx_nufft_amd import _engine as E
+
+    monkeypatch.setattr(E, "_budget", E.TILE_BUDGET)
+    for w, sigma, msub in ((9, 1.25, 1024), (7, 1.25, 64), (9, 2.0, 64)):
+        assert E.spread_msub(E.spread_bins(3, w, [18, 30, 24], 9203), 9203, sigma) == msub

@@ -114,6 +114,12 @@ def spread_bins(dim, w, n_up, P):
         full = 0.4 if w <= 12 else 1.0
         if w > 14 or P < full * float(n_up[0]) * float(n_up[1]):
             return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
+    if dim == 3 and w == 5:
+        # grids smaller than a tile, crowded: 137203 points on 12 x 20 x 10 105 us
+        # with the matrix cores at best, 77 with LDS; 2e4 points 52 and 75
+        cells = float(n_up[0]) * float(n_up[1]) * float(n_up[2])
+        if cells < 4096 and P > 25 * cells:
+            return make_bins(dim, w, n_up, cell_bytes=SPREAD_CELL_BYTES)
     bins = make_bins(dim, w, n_up, m=[max(1, min(17 - w, int(k))) for k in n_up])
     # subproblems: one for each bin with points, and one more for every 1024
     if bins.nbins > 1 << 27 or min(bins.nbins, P) + P // MSUB + MSUB >= 1 << 24:
@@ -133,11 +139,18 @@ def spread_msub(bins, P, sigma=2.0):
     that join the subproblems: w = 9 at sigma = 1.25 on 18 x 30 x 24, 9e3 / 1e5
     points, 9.2e-6 / 1.22e-5 from 64 bits with short ones, 6.7e-6 / 8.1e-6 with
     MSUB and 7.3e-6 / 9.1e-6 in LDS tiles (47 / 76, 71 / 148 and 188 / 333 us);
-    at w = 7 the kernel's own 9.9e-5 hides it."""
+    at w = 7 the kernel's own 9.9e-5 hides it. In 2D no cell takes the edges of
+    more than 500 subproblems on average, or the atomics wait for each other:
+    3 vectors of 63371 points on 10 x 36, w = 5, 63 us with 64, 39 with 128, of
+    5e5 points 153 with 256, 88 to 108 with 512 and more (LDS tiles 50 and 99)."""
     dim, w = bins.dim, bins.w
     if (sigma < 2.0 and w >= 8) or dim == 1 or max(bins.m[d] + w - 1 for d in range(dim)) > 16:
         return MSUB
-    return max(64, min(MSUB, (P // (2048 if dim == 2 else 512) + 63) // 64 * 64))
+    least = 64
+    if dim == 2:
+        cells = float(bins.n[0]) * float(bins.n[1])
+        least = max(64, math.ceil(P * 256 / (500.0 * cells) / 64) * 64)
+    return min(MSUB, max(least, (P // (2048 if dim == 2 else 512) + 63) // 64 * 64))
 
 
 def key_bits(bins):

@@ -407,3 +407,18 @@ def test_subproblem_size_follows_sigma(clib, monkeypatch):
     monkeypatch.setattr(E, "_budget", E.TILE_BUDGET)
     for w, sigma, msub in ((9, 1.25, 1024), (7, 1.25, 64), (9, 2.0, 64)):
         assert E.spread_msub(E.spread_bins(3, w, [18, 30, 24], 9203), 9203, sigma) == msub
+
+
+def test_spread_tiles_on_tiny_grids(clib, monkeypatch):
+    """Small grids with many points: 2D subproblems grow with the points a cell
+    takes, 3D ones at w = 5 keep the LDS bins."""
+    from mlx_nufft_amd import _engine as E
+
+    monkeypatch.setattr(E, "_budget", E.TILE_BUDGET)
+    for n, P, msub in (([10, 36], 5000, 64), ([10, 36], 63371, 128), ([10, 36], 500_000, 768),
+                       ([256, 256], 500_000, 256), ([10, 36], 10_000_000, 1024)):
+        bins = E.spread_bins(2, 5, n, P)
+        assert max(bins.m) + 4 <= 16 and E.spread_msub(bins, P) == msub
+    for P, m in ((20_000, [12, 12, 10]), (137_203, [12, 13, 10])):
+        assert list(E.spread_bins(3, 5, [12, 20, 10], P).m) == m
+    assert list(E.spread_bins(3, 6, [12, 20, 12], 137_203).m) == [11, 11, 11]

@@ -800,7 +800,10 @@ def zgather_preferred(P, w, n_up, sigma=2.0):
     taps. Measured, us, z-gather / tiles: 384 x 400 x 432, 2e6 points, w = 4
     341 / 266, w = 5 349 / 420, w = 8 439 / 866; 200 x 192 x 180, 1.4e6, w = 4
     93 / 67, w = 5 98 / 75, w = 6 104 / 104, w = 8 141 / 235; 1.1e7, w = 5
-    555 / 672. (Below 2^18 points the w <= 5 difference is some us.)
+    555 / 672. (Below 2^18 points the w <= 5 difference is some us.) On grids
+    stored with extents the tiles have all points up to w = 5 there: 1.7e6 on
+    50 x 160 x 72, w = 5, 157 / 104, 5.9e6 on 90 x 100 x 120 412 / 241, 2.5e5 on
+    54 x 50 x 72, w = 4, 73 / 39; 57600 on 50 x 160 x 72, w = 5, 38 / 40.
     Between the factors the other gathers read the grid in fp32, so there the
     z-gather's split operands need the weights that make up for them
     (zgather_stable), and below sigma = 2 they do not: 2e6 points on 360^3 at
@@ -809,6 +812,8 @@ def zgather_preferred(P, w, n_up, sigma=2.0):
     cells = float(n_up[0]) * float(n_up[1]) * float(n_up[2])
     if cells >= 2.0 ** 25:
         return ratio >= (1.5 if sigma >= 2.0 else 5.0)
+    if w <= 5 and (n_up[0] % 8 or n_up[1] % 8):
+        return False
     if w <= 5 and P >= 1 << 18 and (w < 5 or P < 1.2 * cells):
         return False
     return ratio >= 5.0

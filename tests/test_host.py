@@ -422,3 +422,15 @@ def test_spread_tiles_on_tiny_grids(clib, monkeypatch):
     for P, m in ((20_000, [12, 12, 10]), (137_203, [12, 13, 10])):
         assert list(E.spread_bins(3, 5, [12, 20, 10], P).m) == m
     assert list(E.spread_bins(3, 6, [12, 20, 12], 137_203).m) == [11, 11, 11]
+
+
+def test_zgather_rule_on_extents():
+    """Up to w = 5 the z-gather serves its own grids and those of 2^25 cells or
+    more; off its blocks the tiles have the smaller ones."""
+    from mlx_nufft_amd import _engine as E
+
+    for n, P, w, want in (([50, 160, 72], 1_728_000, 5, False), ([54, 50, 72], 249_479, 4, False),
+                          ([54, 50, 72], 249_479, 6, True), ([48, 48, 72], 249_479, 4, True),
+                          ([200, 192, 180], 11_000_000, 5, True),
+                          ([390, 400, 432], 3_000_000, 5, True)):
+        assert E.zgather_preferred(P, w, n) == want, (n, P, w)

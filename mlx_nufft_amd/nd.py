@@ -140,7 +140,7 @@ class _PointsND:
             # w = 4: 209 us without it, 294 with). On the sweep's own grids, where
             # spread-out sets are worth far more, it goes on looking.
             if self._ext:
-                self._ext = None
+                self._ext, self._extsweep = None, False
             else:
                 self._watch = True
             self.pts = None
@@ -151,18 +151,22 @@ class _PointsND:
 
     def _route_by_count(self):
         """What depends on the number of points: the tiles of a spread, and
-        whether they take many points over from the VALU y-sweep (not under
-        stream capture, where their subproblem count cannot be read back)."""
+        whether they take many points over from the VALU y-sweep or on extents
+        (not under stream capture, where their subproblem count cannot be read
+        back)."""
         valu = self._ybins is not None and not self._ymfma
-        key = (self.P, valu and torch.cuda.is_current_stream_capturing())
-        if key == self._routed:
+        capturing = bool(valu or self._ext) and torch.cuda.is_current_stream_capturing()
+        if (self.P, capturing) == self._routed:
             return
-        self._routed = key
+        self._routed = (self.P, capturing)
         if self._cell_bytes == E.SPREAD_CELL_BYTES:
             self.bins = E.spread_bins(self.dim, self.w, self.n_up, self.P)
         self._ysweep = self._ybins is not None and (
             self._ymfma or self.spread_method == "od"
-            or not E.tiles_beat_ysweep(self.bins, self.w, self.P) or key[1])
+            or not E.tiles_beat_ysweep(self.bins, self.w, self.P) or capturing)
+        self._extsweep = self._ext is not None and (
+            self._zgather_points or capturing
+            or not E.tiles_beat_extents(self.w, self.n_up, self._ext, self.P))
 
     # the z-sweep point state is built in the spread's key order unless set
     _zgather_points = False
@@ -213,7 +217,7 @@ class _PointsND:
         to look at once it has time; tiles builds the tiles' state."""
         tm = self._timer()
         load = None
-        if (self._zsweep or self._ext or self._ysweep) and not tiles:
+        if (self._zsweep or self._extsweep or self._ysweep) and not tiles:
             load = self._set_sweep_points(x64, tm, building)
             if load is not None and not building and not self._uncrowded(load, repoint=True):
                 self.pts = None

@@ -355,3 +355,21 @@ def test_crowding_rule_2d_near_break_even(mn):
         v = v / np.linalg.norm(v, axis=0) * np.linspace(-np.pi, np.pi, per, endpoint=False)
         x = tuple(np.ascontiguousarray(a.reshape(-1)[:M]) for a in v)
         assert mn.Type1PlanND(x, (1024, 1024), eps=1e-6).pts.kind == kind
+
+
+def test_dense_narrow_kernels_on_extents(mn):
+    """Up to w = 4 dense sets on small grids stored with extents go to the tiles
+    by their number, on re-pointing as on a new plan."""
+    print("case dense narrow extents", flush=True)
+    rng = np.random.default_rng(44)
+    N, cells = (25, 80, 36), 50 * 160 * 72
+    thin, dense = _pts(rng, cells // 4), _pts(rng, cells)
+    for eps, kind in ((1e-3, "tiles"), (1e-4, "zsweep")):
+        p = mn.Type1PlanND(dense, N, eps=eps)
+        assert p.n_up == [50, 160, 72] and p.pts.kind == kind
+        for x, k in ((thin, "zsweep"), (dense, kind)):
+            p.set_sources(x)
+            assert p.pts.kind == k and (p._store() is None) == (k == "tiles")
+            c = _cplx(rng, x[0].size)
+            ref = mn.Type1PlanND(x, N, eps=eps, spread_method="gm").execute(c)
+            assert np.linalg.norm(p.execute(c) - ref) <= 3e-6 * np.linalg.norm(ref)

@@ -99,7 +99,10 @@ def spread_bins(dim, w, n_up, P):
     cost w^dim, but smaller tiles flush more halo cells. So the matrix cores
     take 3D from w = 5 (us, LDS / matrix cores: 1e6 points on 200 x 180 x 160,
     w = 4: 191 / 219; on 240^3 7e3 to 1.4e6 points, w = 5: 110 / 57 to
-    401 / 373, w = 7: 178 / 69 to 798 / 563, w = 12: 763 / 135 to 7928 / 3576)
+    401 / 373, w = 7: 178 / 69 to 798 / 563, w = 12: 763 / 135 to 7928 / 3576;
+    at w = 5 dense sets that are spread out pay for what crowded ones gain: 4
+    points a cell on 50 x 30 x 180 282 / 324, but 5e6 radial ones on 256^3
+    4629 / 1493)
     and 2D from w = 5 where the points fill the grid (2000^2, w = 6: 0.3
     points per cell 90 / 101, 0.6 143 / 101, 2.4 506 / 281; w = 12: 0.3
     272 / 387, 0.6 505 / 408); wider 2D kernels leave bins of 4 cells or fewer
